@@ -12,6 +12,7 @@
 #include <type_traits>
 
 #include "attn_core.h"
+#include "attn_f32.h"
 #include "launch_util.h"
 
 namespace vfk {
@@ -29,7 +30,8 @@ struct RpbArgs {
   float c2;     // softmax_scale * log2(e)
   float inv_scale;  // 1 / softmax_scale: bias and mask in raw score units
   int bidir, causal, offset_pos;  // offset added for rel > 0 (bidirectional)
-  int lut_len;  // ntiles * kBN + kBM (LDS bias table entries)
+  int lut_len;  // ntiles * kBN + kBM (LDS bias table entries); fp32: > 0 when there is a table
+  int lut_sat;  // fp32: distance from which the bucket no longer changes
   StepFn step;
   // packed sequences (nullptr: the padded batch): "batch" b is sequence b,
   // tokens cu[b] .. cu[b + 1] - 1 of [T, H, D] tensors (strides [.][1] =
@@ -342,64 +344,107 @@ __global__ __launch_bounds__(256, 4) void rpb_fwd_kernel(RpbArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// fp32 kernel: one thread per query row, exact fp32 arithmetic throughout.
+// fp32 kernel (attn_f32.h): the bias of every relative position the workgroup
+// meets, clamped to the distance from which the bucket no longer changes, sits
+// in an LDS table in log2 units; a bucket function that changes further out
+// than kF32MaxLut is evaluated per score.
 // ---------------------------------------------------------------------------
 template <int MASK>
-__global__ __launch_bounds__(64) void rpb_fwd_f32_kernel(RpbArgs a) {
-  __shared__ float Kt[64][kHD + 1];
-  __shared__ float Vt32[64][kHD + 1];
-  const int nqt = (a.Lq + 63) / 64;
-  const int qt = blockIdx.x % nqt;
-  const int bh = blockIdx.x / nqt;
-  const int h = bh % a.H, b = bh / a.H;
-  const int qrow = qt * 64 + threadIdx.x;
-  const bool qvalid = qrow < a.Lq;
-  const float* Qp = reinterpret_cast<const float*>(a.q) + b * a.qs[0] + h * a.qs[1];
-  const float* Kp = reinterpret_cast<const float*>(a.k) + b * a.ks[0] + h * a.ks[1];
-  const float* Vp = reinterpret_cast<const float*>(a.v) + b * a.vs[0] + h * a.vs[1];
-  float qv[kHD], acc[kHD];
-#pragma unroll
-  for (int d = 0; d < kHD; ++d) {
-    qv[d] = qvalid ? Qp[(int64_t)qrow * a.qs[2] + d] : 0.f;
-    acc[d] = 0.f;
+struct RpbF32Policy {
+  const RpbArgs* a;
+  const float* lut;   // bias of rel = lo + index, or nullptr
+  int lo, hi;         // rel is clamped to lo .. hi
+  int qrow, h;        // the lane's query row
+  int64_t mrow;       // mask offset of this (batch, head)
+  float* maskt;       // MASK_KEY: the wave's 64 mask values of the chunk
+  bool skip;          // MASK_KEY: chunks that are masked away entirely are left out
+  __device__ bool chunk(int key0) {
+    if (MASK != MASK_KEY) return true;
+    const int lane = threadIdx.x & 63, j = key0 + lane;
+    const float v = j < a->Lk ? mask_l2(ld_f(a->mask, a->mask_dt, mrow + (int64_t)j * a->ms[3])) : -3.0e38f;
+    // masked by 1e30 beside a key of the row that is not: its probability is 0
+    if (skip && __builtin_amdgcn_ballot_w64(!(v <= -1.0e30f)) == 0ull) return false;
+    __builtin_amdgcn_wave_barrier();
+    maskt[lane] = v;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    return true;
   }
-  float m = -INFINITY, l = 0.f;
-  int kend = a.Lk;
-  if (a.causal) kend = min(kend, min(qt * 64 + 64, a.Lq));
-  for (int key0 = 0; key0 < kend; key0 += 64) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < 64 * kHD; e += 64) {
-      const int r = e / kHD, d = e % kHD;
-      const int j = key0 + r;
-      Kt[r][d] = j < a.Lk ? Kp[(int64_t)j * a.ks[2] + d] : 0.f;
-      Vt32[r][d] = j < a.Lk ? Vp[(int64_t)j * a.vs[2] + d] : 0.f;
-    }
-    __syncthreads();
-    const int nk = min(64, kend - key0);
-    for (int r = 0; r < nk; ++r) {
-      const int j = key0 + r;
-      if (a.causal && j > qrow) break;
-      float s = 0.f;
+  __device__ void load(int kb, int key, f32x4_t& b) const {
+    f32x4_t mv = {};
+    if (MASK == MASK_KEY) mv = *reinterpret_cast<const f32x4_t*>(maskt + 16 * kb + 4 * ((threadIdx.x & 63) >> 4));
 #pragma unroll
-      for (int d = 0; d < kHD; ++d) s += qv[d] * Kt[r][d];
-      s = s * a.c2;
-      if (a.table) s += ld_f(a.table, a.table_dt, rpb_bucket(a, j - qrow) * a.tb0 + h * a.tb1) * VFK_LOG2E;
-      if (MASK != MASK_NONE)
-        s += mask_l2(ld_f(a.mask, a.mask_dt, b * a.ms[0] + h * a.ms[1] + (int64_t)qrow * a.ms[2] + (int64_t)j * a.ms[3]));
-      const float mn = fmaxf(m, s);
-      const float alpha = exp2f(m - mn);
-      const float p = exp2f(s - mn);
-      l = l * alpha + p;
-#pragma unroll
-      for (int d = 0; d < kHD; ++d) acc[d] = acc[d] * alpha + p * Vt32[r][d];
-      m = mn;
+    for (int r = 0; r < 4; ++r) {
+      const int rel = key + r - qrow;
+      float x = 0.f;
+      if (a->table) {
+        if (lut) x = lut[min(max(rel, lo), hi) - lo];
+        else x = ld_f(a->table, a->table_dt, rpb_bucket(*a, rel) * a->tb0 + h * a->tb1) * VFK_LOG2E;
+      }
+      if (MASK == MASK_KEY) x += mv[r];
+      if (MASK == MASK_FULL)
+        x += mask_l2(ld_f(a->mask, a->mask_dt, mrow + (int64_t)min(qrow, a->Lq - 1) * a->ms[2] +
+                                                   (int64_t)min(key + r, a->Lk - 1) * a->ms[3]));
+      b[r] = x;
     }
   }
-  if (!qvalid) return;
-  float* op = reinterpret_cast<float*>(a.o) + b * a.os[0] + h * a.os[1] + (int64_t)qrow * a.os[2];
-  const float inv = l > 0.f ? 1.0f / l : 0.f;
-#pragma unroll
-  for (int d = 0; d < kHD; ++d) op[d] = acc[d] * inv;
+  __device__ float score(float s, float b) const { return __builtin_fmaf(s, a->c2, b); }
+};
+
+template <int MASK, bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void rpb_fwd_f32_kernel(RpbArgs a) {
+  __shared__ __align__(16) F32Merge sm;
+  __shared__ __align__(16) float maskt[MASK == MASK_KEY ? kF32Waves * 64 : 4];
+  __shared__ int16_t thr[VFK_MAX_THR];
+  extern __shared__ float lutf[];
+  const int nqt = (a.Lq + kF32Rows - 1) / kF32Rows;
+  const int work = xcd_remap(blockIdx.x, gridDim.x);
+  const int bh = work / nqt, h = bh % a.H, b = bh / a.H;
+  const int t = threadIdx.x;
+  F32Args f;
+  f.q = reinterpret_cast<const float*>(a.q) + b * a.qs[0] + h * a.qs[1];
+  f.k = reinterpret_cast<const float*>(a.k) + b * a.ks[0] + h * a.ks[1];
+  f.v = reinterpret_cast<const float*>(a.v) + b * a.vs[0] + h * a.vs[1];
+  f.o = reinterpret_cast<float*>(a.o) + b * a.os[0] + h * a.os[1];
+  f.qs = a.qs[2]; f.ks = a.ks[2]; f.vs = a.vs[2]; f.os = a.os[2];
+  f.q0 = (work % nqt) * kF32Rows;
+  f.nq = f.nstore = a.Lq;
+  f.coff = 0;
+  f.kend = CAUSAL ? min(a.Lk, min(f.q0 + kF32Rows, a.Lq)) : a.Lk;
+  RpbF32Policy<MASK> pol;
+  pol.a = &a;
+  pol.lut = nullptr;
+  pol.lo = pol.hi = 0;
+  pol.qrow = f.q0 + (t & 15);
+  pol.h = h;
+  pol.mrow = b * a.ms[0] + h * a.ms[1];
+  pol.maskt = maskt + (MASK == MASK_KEY ? 64 * (t >> 6) : 0);
+  pol.skip = false;
+  if (MASK == MASK_KEY && !CAUSAL) {
+    // some key well above -1e30: usually among the first 256
+    for (int j0 = 0; j0 < a.Lk && !pol.skip; j0 += 256) {
+      const int j = j0 + t;
+      pol.skip = __syncthreads_or(
+          j < a.Lk && mask_l2(ld_f(a.mask, a.mask_dt, pol.mrow + (int64_t)j * a.ms[3])) > -1.0e29f);
+    }
+  }
+  if (a.lut_len > 0) {  // the launch holds an LDS table
+    pol.lo = min(max(-(f.q0 + kF32Rows - 1), -a.lut_sat), a.lut_sat);
+    pol.hi = min(max(f.kend - 1 - f.q0, -a.lut_sat), a.lut_sat);
+    pol.lut = lutf;
+    for (int e = t; e < a.step.nthr; e += 256) thr[e] = a.step.thr[e];
+    __syncthreads();
+    for (int e = t; e <= pol.hi - pol.lo; e += 256) {
+      const int rel = pol.lo + e;
+      int bk = step_eval_lds(a.step, thr, rel < 0 ? -rel : (a.bidir ? rel : 0));
+      if (a.bidir && rel > 0) bk += a.offset_pos;
+      bk = min(max(bk, 0), a.total_buckets - 1);
+      lutf[e] = ld_f(a.table, a.table_dt, bk * a.tb0 + h * a.tb1) * VFK_LOG2E;
+    }
+    __syncthreads();
+  }
+  f32_attend<CAUSAL>(f, pol, sm);
 }
 
 }  // namespace vfk
@@ -483,6 +528,29 @@ static int rpb_launch(RpbArgs& a, int mode, int dt, hipStream_t st, const char* 
   return launch_status(name);
 }
 
+static int rpb_f32_launch(RpbArgs& a, int mode, hipStream_t st, const char* name) {
+  const int64_t grid = (int64_t)a.B * a.H * ceil_div(a.Lq, kF32Rows);
+  if (grid >= (1ll << 31)) return set_error(VFK_ERR_UNSUPPORTED, "%s: sizes too large", name);
+  a.lut_len = 0;
+  if (a.table) {
+    a.lut_sat = std::min(step_saturates_at(a.step), std::max(a.Lq, a.Lk));
+    if (a.lut_sat <= kF32MaxLut) a.lut_len = std::min(2 * a.lut_sat + 1, a.Lk + kF32Rows - 1);
+  }
+  const size_t lds = (size_t)a.lut_len * 4;
+#define VFK_RPB_F32(M, C) \
+  hipLaunchKernelGGL((rpb_fwd_f32_kernel<M, C>), dim3((unsigned)grid), dim3(256), lds, st, a)
+#define VFK_RPB_F32_M(M) \
+  if (a.causal) VFK_RPB_F32(M, true); else VFK_RPB_F32(M, false);
+  switch (mode) {
+    case MASK_NONE: VFK_RPB_F32_M(MASK_NONE) break;
+    case MASK_KEY: VFK_RPB_F32_M(MASK_KEY) break;
+    default: VFK_RPB_F32_M(MASK_FULL) break;
+  }
+#undef VFK_RPB_F32_M
+#undef VFK_RPB_F32
+  return launch_status(name);
+}
+
 extern "C" int vfk_flash_rpb_fwd(const vfk_tensor* q, const vfk_tensor* k,
                                  const vfk_tensor* v, const vfk_tensor* rpb_table,
                                  int32_t num_buckets, int32_t max_distance,
@@ -530,15 +598,7 @@ extern "C" int vfk_flash_rpb_fwd(const vfk_tensor* q, const vfk_tensor* k,
   if (Lk == 0)
     return set_error(VFK_ERR_INVALID, "vfk_flash_rpb_fwd: no keys");
   hipStream_t st = (hipStream_t)stream;
-  if (dt == VFK_F32) {
-    const int nqt = ceil_div(Lq, 64);
-    dim3 grid((unsigned)(nqt * B * H));
-    if (mode == MASK_NONE)
-      hipLaunchKernelGGL(rpb_fwd_f32_kernel<MASK_NONE>, grid, dim3(64), 0, st, a);
-    else
-      hipLaunchKernelGGL(rpb_fwd_f32_kernel<MASK_FULL>, grid, dim3(64), 0, st, a);
-    return launch_status(name);
-  }
+  if (dt == VFK_F32) return rpb_f32_launch(a, mode, st, name);
   return rpb_launch(a, mode, dt, st, name);
 }
 
