@@ -13,7 +13,10 @@
 // from the exact fp32 formula); the inner loop reads it with immediate offsets.
 #include <math.h>
 
+#include <algorithm>
+
 #include "attn_core.h"
+#include "attn_f32.h"
 #include "launch_util.h"
 
 namespace vfk {
@@ -296,69 +299,108 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
   }
 }
 
-// fp32: one thread per query row.
-__global__ __launch_bounds__(64) void deberta_gather_f32_kernel(DebArgs a) {
-  __shared__ float Kt[64][kHD + 1];
-  __shared__ float Vt32[64][kHD + 1];
-  const int nqt = (a.M + 63) / 64;
-  const int qt = blockIdx.x % nqt;
-  const int bh = blockIdx.x / nqt;
-  const int h = bh % a.H, b = bh / a.H;
-  const int qrow = qt * 64 + threadIdx.x;
-  const int len = a.seq_lengths ? min(max(a.seq_lengths[b], 0), a.N) : a.N;
-  const bool qstore = qrow < a.M;
-  const bool qvalid = qrow < min(len, a.M);
-  const float* Qp = reinterpret_cast<const float*>(a.q) + b * a.qs[0] + h * a.qs[1];
-  const float* Kp = reinterpret_cast<const float*>(a.k) + b * a.ks[0] + h * a.ks[1];
-  const float* Vp = reinterpret_cast<const float*>(a.v) + b * a.vs[0] + h * a.vs[1];
-  const float* PK = reinterpret_cast<const float*>(a.pk);
-  const float* PQ = reinterpret_cast<const float*>(a.pq);
-  float qv[kHD], acc[kHD];
-#pragma unroll
-  for (int d = 0; d < kHD; ++d) {
-    qv[d] = qvalid ? Qp[(int64_t)qrow * a.qs[2] + d] : 0.f;
-    acc[d] = 0.f;
-  }
-  float m = -INFINITY, l = 0.f;
-  int kend = len;
-  if (a.causal) kend = min(kend, min(qt * 64 + 64, a.M) + (a.N - a.M));
-  for (int key0 = 0; key0 < kend; key0 += 64) {
-    __syncthreads();
-    for (int e = threadIdx.x; e < 64 * kHD; e += 64) {
-      const int r = e / kHD, d = e % kHD;
-      const int j = key0 + r;
-      Kt[r][d] = j < kend ? Kp[(int64_t)j * a.ks[2] + d] : 0.f;
-      Vt32[r][d] = j < kend ? Vp[(int64_t)j * a.vs[2] + d] : 0.f;
-    }
-    __syncthreads();
-    if (!qvalid) continue;
-    const int nk = min(64, kend - key0);
-    for (int r = 0; r < nk; ++r) {
-      const int j = key0 + r;
-      if (a.causal && j > qrow + (a.N - a.M)) break;
-      float s = 0.f;
-#pragma unroll
-      for (int d = 0; d < kHD; ++d) s += qv[d] * Kt[r][d];
-      const int c = deb_index(a, qrow - j);
-      if (PK) s += PK[b * a.pks[0] + h * a.pks[1] + (int64_t)qrow * a.pks[2] + (int64_t)c * a.pks[3]];
-      if (PQ) s += PQ[b * a.pqs[0] + h * a.pqs[1] + (int64_t)j * a.pqs[2] + (int64_t)c * a.pqs[3]];
-      s *= a.c2;
-      const float mn = fmaxf(m, s);
-      const float alpha = exp2f(m - mn);
-      const float p = exp2f(s - mn);
-      l = l * alpha + p;
-#pragma unroll
-      for (int d = 0; d < kHD; ++d) acc[d] = acc[d] * alpha + p * Vt32[r][d];
-      m = mn;
-    }
-  }
-  if (!qstore) return;
-  float* op = reinterpret_cast<float*>(a.o) + b * a.os[0] + h * a.os[1] + (int64_t)qrow * a.os[2];
-  const float inv = (qvalid && l > 0.f) ? 1.0f / l : 0.f;
-#pragma unroll
-  for (int d = 0; d < kHD; ++d) op[d] = acc[d] * inv;
-}
+// fp32 (attn_f32.h): the column c(i - j) of every distance the workgroup
+// meets, clamped to the distance from which it no longer changes, comes from
+// an LDS table (or is evaluated per score: linear buckets, and functions that
+// change further out than kF32MaxLut); the position terms are gathered from
+// global memory ahead of the score product, which hides them. RUN: c moves by
+// at most 1 per unit of distance and pos_key columns are contiguous, so the
+// lane's four keys of a block lie in four consecutive columns of its row, one
+// 16-byte load in place of four gathers over 16 rows.
+struct DebF32Args {
+  int lut;   // LDS table of c
+  int sat;   // distance from which c no longer changes
+};
 
+template <bool RUN>
+struct DebF32Policy {
+  const DebArgs* a;
+  const int16_t* lut;      // c(lo + index), or nullptr
+  int lo, hi;              // distances are clamped to lo .. hi
+  const float* prow;       // the lane's pos_key row, or nullptr
+  const float* pq;         // pos_query rows of this (batch, head), or nullptr
+  int qrow;                // the lane's query row
+  __device__ bool chunk(int) { return true; }
+  __device__ int column(int d) const {
+    return lut ? lut[min(max(d, lo), hi) - lo] : deb_index(*a, d);
+  }
+  __device__ void load(int, int key, f32x4_t& b) const {
+    int col[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) col[r] = column(qrow - (key + r));
+    b = f32x4_t{};
+    if (prow) {
+      if (RUN) {
+        const int start = min(col[3], 2 * a->span - 4);  // col[3] <= col[2] <= ..
+        const f32x4_t w = ld4(prow + start);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int e = col[r] - start;
+          b[r] = e < 2 ? (e == 0 ? w[0] : w[1]) : (e == 2 ? w[2] : w[3]);
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) b[r] = prow[(int64_t)col[r] * a->pks[3]];
+      }
+    }
+    if (pq) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        b[r] += pq[(int64_t)min(key + r, a->N - 1) * a->pqs[2] + (int64_t)col[r] * a->pqs[3]];
+    }
+  }
+  __device__ float score(float s, float b) const { return (s + b) * a->c2; }
+};
+
+template <bool RUN, bool CAUSAL>
+__global__ __launch_bounds__(256, 2) void deberta_gather_f32_kernel(DebArgs a, DebF32Args x) {
+  __shared__ __align__(16) F32Merge sm;
+  __shared__ int16_t thr[VFK_MAX_THR];
+  extern __shared__ int16_t lutc[];
+  const int nqt = (a.M + kF32Rows - 1) / kF32Rows;
+  const int work = xcd_remap(blockIdx.x, gridDim.x);
+  const int bh = work / nqt, h = bh % a.H, b = bh / a.H;
+  const int t = threadIdx.x;
+  const int len = a.seq_lengths ? min(max(a.seq_lengths[b], 0), a.N) : a.N;
+  F32Args f;
+  f.q = reinterpret_cast<const float*>(a.q) + b * a.qs[0] + h * a.qs[1];
+  f.k = reinterpret_cast<const float*>(a.k) + b * a.ks[0] + h * a.ks[1];
+  f.v = reinterpret_cast<const float*>(a.v) + b * a.vs[0] + h * a.vs[1];
+  f.o = reinterpret_cast<float*>(a.o) + b * a.os[0] + h * a.os[1];
+  f.qs = a.qs[2]; f.ks = a.ks[2]; f.vs = a.vs[2]; f.os = a.os[2];
+  f.q0 = (work % nqt) * kF32Rows;
+  f.nq = min(len, a.M);
+  f.nstore = a.M;
+  f.coff = a.N - a.M;
+  f.kend = CAUSAL ? min(len, min(f.q0 + kF32Rows, a.M) + f.coff) : len;
+  if (f.q0 >= f.nq || f.kend <= 0) {  // no row with a key: uniform exit
+    f32_zero_rows(f);
+    return;
+  }
+  DebF32Policy<RUN> pol;
+  pol.a = &a;
+  pol.lut = nullptr;
+  pol.lo = pol.hi = 0;
+  if (x.lut) {
+    pol.lut = lutc;
+    pol.lo = min(max(f.q0 - (f.kend - 1), -x.sat), x.sat);
+    pol.hi = min(max(f.q0 + kF32Rows - 1, -x.sat), x.sat);
+    for (int e = t; e < a.step.nthr; e += 256) thr[e] = a.step.thr[e];
+    __syncthreads();
+    for (int e = t; e <= pol.hi - pol.lo; e += 256) {
+      const int d = pol.lo + e;
+      const int mag = step_eval_lds(a.step, thr, d < 0 ? -d : d);
+      lutc[e] = (int16_t)min(max((d < 0 ? -mag : mag) + a.span, 0), 2 * a.span - 1);
+    }
+    __syncthreads();
+  }
+  pol.qrow = f.q0 + (t & 15);
+  pol.prow = a.pk ? reinterpret_cast<const float*>(a.pk) + b * a.pks[0] + h * a.pks[1] +
+                        (int64_t)min(pol.qrow, a.M - 1) * a.pks[2]
+                  : nullptr;
+  pol.pq = a.pq ? reinterpret_cast<const float*>(a.pq) + b * a.pqs[0] + h * a.pqs[1] : nullptr;
+  f32_attend<CAUSAL>(f, pol, sm);
+}
 
 // ---------------------------------------------------------------------------
 // Fused form: c2p / p2c computed in the kernel from the per-head projections
@@ -901,6 +943,25 @@ static int check_pos(const vfk_tensor* p, const char* name, const DebArgs& a, in
   return VFK_OK;
 }
 
+static int deb_gather_f32_launch(const DebArgs& a, hipStream_t st, const char* name) {
+  const int64_t grid = (int64_t)a.B * a.H * ceil_div(a.M, kF32Rows);
+  if (grid >= (1ll << 31)) return set_error(VFK_ERR_UNSUPPORTED, "%s: sizes too large", name);
+  DebF32Args x = {};
+  x.sat = std::min(step_saturates_at(a.step), std::max(a.M, a.N));
+  x.lut = a.log_bucket && x.sat <= kF32MaxLut && a.span <= 16384;  // c fits 16 bits
+  const size_t lds = x.lut ? (size_t)std::min(2 * x.sat + 1, a.N + kF32Rows - 1) * 2 : 0;
+  const bool run = a.unit && a.pk && a.pks[3] == 1 && a.span >= 2;
+#define VFK_DEB_F32(R, C) \
+  hipLaunchKernelGGL((deberta_gather_f32_kernel<R, C>), dim3((unsigned)grid), dim3(256), lds, st, a, x)
+  if (a.causal) {
+    if (run) VFK_DEB_F32(true, true); else VFK_DEB_F32(false, true);
+  } else {
+    if (run) VFK_DEB_F32(true, false); else VFK_DEB_F32(false, false);
+  }
+#undef VFK_DEB_F32
+  return launch_status(name);
+}
+
 extern "C" int vfk_flash_deberta_fwd(const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,
                                      const int32_t* seq_lengths, const vfk_tensor* pos_key,
                                      const vfk_tensor* pos_query, int32_t causal, float sm_scale,
@@ -923,11 +984,7 @@ extern "C" int vfk_flash_deberta_fwd(const vfk_tensor* q, const vfk_tensor* k, c
   }
   if (a.B == 0 || a.H == 0 || a.M == 0) return VFK_OK;
   hipStream_t st = (hipStream_t)stream;
-  if (q->dtype == VFK_F32) {
-    const int nqt = ceil_div(a.M, 64);
-    hipLaunchKernelGGL(deberta_gather_f32_kernel, dim3((unsigned)(nqt * a.B * a.H)), dim3(64), 0, st, a);
-    return launch_status("vfk_flash_deberta_fwd");
-  }
+  if (q->dtype == VFK_F32) return deb_gather_f32_launch(a, st, "vfk_flash_deberta_fwd");
   const int ntk = ceil_div(a.N, kBN);
   a.lut_len = ntk * kBN + kBM;
   const size_t lds = (size_t)(kKsElems + kVtElems) * 2 + (size_t)a.lut_len * 2;
