@@ -97,3 +97,27 @@ def test_glu_linear_modernbert_config5_shape(dev):
     assert_elem_close(got[rows], want, torch.bfloat16, "config-5 rows")
     assert torch.isfinite(got.float()).all()
     assert cosine(got[rows], want) >= 0.9999
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M,K,I", [
+    (1, 64, 8), (31, 192, 40), (33, 320, 1152), (224, 768, 1152),       # 32 x 32 tiles, K split unevenly
+    (225, 64, 1152), (257, 128, 1160), (500, 768, 1152), (65, 1024, 8200),  # 64 x 64
+    (4600, 128, 1152), (4700, 128, 1152)])                              # the line to 256 x 128
+def test_glu_linear_tiles(dev, dtype, M, K, I):
+    """Each tile at its edges: K slices that do not divide among the waves,
+    fewer slices than stages, ragged tokens and features; x and w with row
+    strides above K, whose gaps and tails must not enter (they hold NaN). The
+    bound is the one above."""
+    from kernels.fused_glu_mlp import glu_linear
+    print("glu tiles", dtype, M, K, I, flush=True)
+    x, w = _inputs(M, K, I, dtype, M + K + I)
+    xd = torch.full((M, K + 8), float("nan"), dtype=dtype, device=dev)
+    wd = torch.full((2 * I, K + 8), float("nan"), dtype=dtype, device=dev)
+    xd[:, :K], wd[:, :K] = x.to(dev), w.to(dev)
+    out = torch.full((M + 1, I + 8), 7.0, dtype=dtype, device=dev)
+    glu_linear(xd[:, :K], wd[:, :K], "gelu", out=out[:M, :I])
+    assert (out[M] == 7.0).all() and (out[:, I:] == 7.0).all(), "written past the output"
+    y = xd[:, :K].double() @ wd[:, :K].double().t()
+    want = torch.nn.functional.gelu(y[:, :I]) * y[:, I:]
+    assert_elem_close(out[:M, :I], want, dtype, f"glu_linear {M}x{K}x{I}")
