@@ -22,7 +22,7 @@ def binary(entry: str, act: int, a: torch.Tensor, b: torch.Tensor) -> torch.Tens
     if a.dtype != b.dtype:
         raise ValueError("operands must share a dtype")
     a2, b2 = flat2d(a), flat2d(b)
-    out = torch.empty(a2.shape, dtype=a.dtype, device=a.device)
+    out = a.new_empty(a2.shape)
     if out.numel():
         if entry == "vfk_glu_fwd":
             _lib.on_device(entry, dev, int(act), _lib.ref(_lib.desc(a2)),

@@ -18,7 +18,7 @@ def activation(x: torch.Tensor, act_fn: str = "gelu") -> torch.Tensor:
         raise NotImplementedError(f"activation {act_fn!r} is not built")
     dev = _lib.require_gpu(x)
     x2 = flat2d(x)
-    out = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
+    out = x.new_empty(x2.shape)
     if out.numel():
         _lib.on_device("vfk_act_fwd", dev, int(_ACT[act_fn]), _lib.ref(_lib.desc(x2)),
                        _lib.ref(_lib.desc(out)))

@@ -62,7 +62,7 @@ def dense_add_layernorm(x: torch.Tensor, weight: Optional[torch.Tensor], bias: O
     if not in_place:
         r2 = _lib.rows_aligned(r2)
     if out is None:
-        o2 = torch.empty(r2.shape, dtype=x.dtype, device=x.device)
+        o2 = x.new_empty(r2.shape)
     else:
         if out.shape != residual.shape:
             raise ValueError(f"out must be {tuple(residual.shape)}, got {tuple(out.shape)}")

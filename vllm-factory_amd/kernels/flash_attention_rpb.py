@@ -47,7 +47,7 @@ def flash_attention_rpb_final(
         raise ValueError("q, k, v must share a dtype")
     qq, kk, vv = (_lib.rows_aligned(t) for t in (q, k, v))
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        out = q.new_empty(q.shape)
     elif out.shape != q.shape or out.dtype != q.dtype or out.device != q.device:
         raise ValueError("out must match q's shape, dtype and device")
     mask = padding_mask
@@ -94,7 +94,7 @@ def flash_attention_rpb_varlen(
         raise ValueError("q, k, v must share a dtype")
     qq, kk, vv = (_lib.rows_aligned(t) for t in (q, k, v))
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        out = q.new_empty(q.shape)
     elif out.shape != q.shape or out.dtype != q.dtype or out.device != q.device:
         raise ValueError("out must match q's shape, dtype and device")
     cu = cu_seqlens.to(torch.int32).contiguous()

@@ -90,7 +90,7 @@ def flash_deberta_attention(
     pk = pos_key.to(q.dtype) if pos_key is not None else None
     pq = pos_query.to(q.dtype) if pos_query is not None else None
     sl = _seq_lengths(seq_lengths, B, dev)
-    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    out = q.new_empty(q.shape)
     _lib.on_device(
         "vfk_flash_deberta_fwd", dev,
         _lib.ref(_lib.desc(qq)), _lib.ref(_lib.desc(kk)), _lib.ref(_lib.desc(vv)),
@@ -172,7 +172,7 @@ def flash_deberta_attention_fused(
     kr, qr = _rel_tables(key_rel, query_rel, q.dtype, span, chunk_major)
     sl = _seq_lengths(seq_lengths, B, dev)
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        out = q.new_empty(q.shape)
     elif (out.shape != q.shape or out.dtype != q.dtype or out.device != q.device
           or _lib.rows_aligned(out) is not out):
         raise ValueError("out must match q's shape, dtype and device, with contiguous 16-byte rows")
@@ -217,7 +217,7 @@ def flash_deberta_attention_varlen(
     span = position_buckets if position_buckets > 0 else max_relative_distance
     kr, qr = _rel_tables(key_rel, query_rel, q.dtype, span, chunk_major)
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        out = q.new_empty(q.shape)
     elif (out.shape != q.shape or out.dtype != q.dtype or out.device != q.device
           or _lib.rows_aligned(out) is not out):
         raise ValueError("out must match q's shape, dtype and device, with contiguous 16-byte rows")

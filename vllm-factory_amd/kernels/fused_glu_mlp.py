@@ -53,12 +53,12 @@ def glu_linear(x: torch.Tensor, weight: torch.Tensor, act_fn: str = "gelu",
     if weight.dtype != x.dtype:
         raise ValueError("glu_linear: x and weight must share a dtype")
     I = weight.shape[0] // 2
-    x2 = _lib.rows_aligned(x.reshape(-1, K))
+    x2 = _lib.rows_aligned(x if x.dim() == 2 else x.reshape(-1, K))
     w2 = _lib.rows_aligned(weight)
     if out is None:
-        out = torch.empty(x2.shape[0], I, dtype=x.dtype, device=x.device)
+        out = x.new_empty((x2.shape[0], I))
     elif out.shape != (x2.shape[0], I) or out.dtype != x.dtype:
         raise ValueError(f"glu_linear: out must be [{x2.shape[0]}, {I}] {x.dtype}")
     _lib.on_device("vfk_glu_linear_fwd", dev, _act_code(act_fn), _lib.ref(_lib.desc(x2)),
                    _lib.ref(_lib.desc(w2)), _lib.ref(_lib.desc(out)))
-    return out.view(*x.shape[:-1], I)
+    return out if x.dim() == 2 else out.view(*x.shape[:-1], I)

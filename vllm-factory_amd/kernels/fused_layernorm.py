@@ -15,7 +15,7 @@ from . import _lib
 
 
 def _as_2d(x: torch.Tensor, n: int) -> torch.Tensor:
-    x2 = x.reshape(-1, n)
+    x2 = x if x.dim() == 2 else x.reshape(-1, n)
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
     return x2
@@ -28,7 +28,7 @@ def _norm(x: torch.Tensor, n: int, weight: Optional[torch.Tensor], bias: Optiona
     if x.shape[-1] != n:
         raise ValueError(f"last dim {x.shape[-1]} != normalized size {n}")
     x2 = _as_2d(x, n)
-    y = torch.empty(x2.shape, dtype=x.dtype, device=x.device)
+    y = x.new_empty(x2.shape)
     r2 = _as_2d(residual, n) if residual is not None else None
     s2 = torch.empty_like(y) if (residual is not None and want_sum) else None
     w = weight.contiguous() if weight is not None else None
@@ -41,10 +41,10 @@ def _norm(x: torch.Tensor, n: int, weight: Optional[torch.Tensor], bias: Optiona
         _lib.on_device("vfk_layernorm_fwd", dev, _lib.ref(_lib.desc(x2)), _lib.ref(_lib.desc(r2)),
                        _lib.ref(_lib.desc(w)), _lib.ref(_lib.desc(b)), float(eps),
                        _lib.ref(_lib.desc(y)), _lib.ref(_lib.desc(s2)))
-    y = y.view(x.shape)
-    if s2 is not None:
-        return y, s2.view(x.shape)
-    return y
+    if x.dim() != 2:
+        y = y.view(x.shape)
+        s2 = s2.view(x.shape) if s2 is not None else None
+    return (y, s2) if s2 is not None else y
 
 
 class FusedLayerNorm(torch.nn.Module):

@@ -35,13 +35,19 @@ def rope_table(theta: float, positions: int, device: torch.device) -> torch.Tens
     (vfk_rope_table), cached per (theta, size bucket, device) the way the HF
     rotary module caches its tables."""
     n = max(256, 1 << (max(positions, 1) - 1).bit_length())
-    key = (float(theta), n, torch.device(device))
+    key = (float(theta), n, device if isinstance(device, torch.device) else torch.device(device))
     t = _ROPE_TABLES.get(key)
     if t is None:
         t = torch.empty(n, 32, 2, dtype=torch.float32, device=device)
         _lib.on_device("vfk_rope_table", torch.device(device), float(theta), int(n), t.data_ptr())
         _ROPE_TABLES[key] = t
     return t
+
+
+def _bytes_of(mask: torch.Tensor) -> torch.Tensor:
+    """A key mask as contiguous uint8; booleans are bytes already (no pass over them)."""
+    mask = mask.view(torch.uint8) if mask.dtype == torch.bool else mask.to(torch.uint8)
+    return mask.contiguous()
 
 
 def varlen_rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
@@ -60,12 +66,12 @@ def varlen_rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
         cu_seqlens = cu_seqlens.contiguous()
     qq, kk, vv = (_lib.rows_aligned(t) for t in (q, k, v))
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        out = q.new_empty(q.shape)
     kv_ptr = None
     if key_valid is not None:
         if key_valid.numel() != q.shape[0]:
             raise ValueError("key_valid must have one entry per token")
-        key_valid = key_valid.to(torch.uint8).contiguous()
+        key_valid = _bytes_of(key_valid)
         kv_ptr = key_valid.data_ptr()
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(q.shape[-1])
     tab_ptr, tab_n = None, 0
@@ -76,7 +82,7 @@ def varlen_rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     ws_bytes = int(_lib.load().vfk_varlen_attn_workspace_bytes(
         _lib.dtype_code(q.dtype), int(q.shape[0]), int(q.shape[1]), int(rope),
         int(cu_seqlens.numel() - 1), int(max_seqlen)))
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device) if ws_bytes else None
+    ws = q.new_empty(ws_bytes, dtype=torch.uint8) if ws_bytes else None
     _lib.on_device(
         "vfk_varlen_attn_fwd", dev,
         _lib.ref(_lib.desc(qq)), _lib.ref(_lib.desc(kk)), _lib.ref(_lib.desc(vv)),
@@ -150,12 +156,12 @@ def varlen_rope_attention_krot(qkv: RotatedQKV, cu_seqlens: torch.Tensor, max_se
     if not cu_seqlens.is_contiguous():
         cu_seqlens = cu_seqlens.contiguous()
     if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+        out = q.new_empty(q.shape)
     kv_ptr = None
     if key_valid is not None:
         if key_valid.numel() != q.shape[0]:
             raise ValueError("key_valid must have one entry per token")
-        key_valid = key_valid.to(torch.uint8).contiguous()
+        key_valid = _bytes_of(key_valid)
         kv_ptr = key_valid.data_ptr()
     tab = rope_table(qkv.rope_theta, int(max_seqlen), dev)
     _lib.on_device(
