@@ -510,6 +510,31 @@ int vfk_glu_fwd(int32_t act, const vfk_tensor* a, const vfk_tensor* b,
 int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_tensor* w,
                        vfk_tensor* out, void* stream);
 
+/* One ModernBERT layer over packed sequences (models/modernbert/
+ * modernbert_encoder.py:289-352), for few tokens: all of its kernels are
+ * enqueued by one call, the products run on 32 x 32 and 64 x 128 tiles.
+ *   x1 = x + pending; att = attention(LayerNorm(x1) wqkv^T);
+ *   x_out = x1 + att wo^T; pending_out = GLU(LayerNorm(x_out) wi^T) wo_mlp^T
+ * with GLU = GELU(first half) * second half. pending NULL: x1 = x; attn_norm
+ * NULL (layer 0, pending NULL too): no first LayerNorm. x, pending, x_out,
+ * pending_out [T, D] contiguous; norms [D]; wqkv [3D, D], wo [D, D], wi
+ * [2I, D], wo_mlp [D, I] with 16-byte aligned rows; all bf16 or all fp16; D
+ * and I multiples of 64, D / 64 heads. x_out must not be x. The attention's
+ * arguments are those of vfk_varlen_attn_fwd. The workspace takes
+ * vfk_modernbert_layer_workspace_bytes and may be shared by the layers of one
+ * stream. */
+int64_t vfk_modernbert_layer_workspace_bytes(int32_t dtype, int64_t tokens, int32_t hidden,
+                                             int32_t inter, int32_t num_seqs, int32_t max_seqlen);
+int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* pending,
+                             const vfk_tensor* attn_norm, const vfk_tensor* wqkv,
+                             const vfk_tensor* wo, const vfk_tensor* mlp_norm,
+                             const vfk_tensor* wi, const vfk_tensor* wo_mlp, float eps,
+                             const int32_t* cu_seqlens, int32_t num_seqs, int32_t max_seqlen,
+                             int32_t window, const float* rope_cos_sin, int32_t rope_positions,
+                             const uint8_t* key_valid, float softmax_scale, void* workspace,
+                             int64_t workspace_bytes, vfk_tensor* x_out, vfk_tensor* pending_out,
+                             void* stream);
+
 /* Dense projection, bias, residual add and LayerNorm in one kernel:
  *   out = LayerNorm(round(x w^T + bias) + residual) * ln_weight + ln_bias,
  * DeBERTa's post-LN output blocks (DebertaV2SelfOutput.forward and

@@ -1,0 +1,97 @@
+"""The ModernBERT layers of few tokens (vfk_modernbert_layer_fwd) against the
+same layers in 64 bits, at the edges of its tiles: 32 x 32 tiles with the norm
+in front (few tokens), 64 x 128 with a separate one, ragged tokens, K slices
+that do not divide among the waves, a width that the fused norm does not hold.
+
+Bound: each of a layer's seven 16-bit roundings is off by 2^-9 (bf16) of its
+value at most, 2^-9 / sqrt(3) in the mean, so two layers stay within
+sqrt(14) * 2^-9 / sqrt(3) = 4.2e-3 of the residual stream's norm; fp16 has
+three more bits. Twice that is allowed."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from encoders import modernbert as mb
+from oracle import attention as oa
+
+pytestmark = pytest.mark.gpu
+
+
+def _weights(D, I, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    rnd = lambda *s: (torch.randn(*s, generator=g) / s[-1] ** 0.5).to(dtype)
+    ones = lambda: (1 + 0.1 * torch.randn(D, generator=g)).to(dtype)
+    layers = [mb.ModernBertLayerWeights(rnd(3 * D, D), rnd(D, D), rnd(2 * I, D), rnd(D, I),
+                                        None if i == 0 else ones(), ones()) for i in range(2)]
+    return mb.ModernBertWeights(D, D // 64, I, torch.randn(100, D, generator=g).to(dtype), ones(), layers, ones())
+
+
+def _want(ids, cu, w):
+    ln = lambda x, g: F.layer_norm(x, (w.hidden,), g.double(), None, w.eps)
+    x = ln(w.emb[ids].double(), w.emb_norm)
+    for i, lw in enumerate(w.layers):
+        h = x if lw.attn_norm is None else ln(x, lw.attn_norm)
+        q, k, v = (h @ lw.wqkv.double().t()).view(-1, 3, w.heads, 64).unbind(1)
+        glob = i % w.global_every == 0
+        a = oa.varlen_attention(q, k, v, cu, -1 if glob else w.window, w.theta_global if glob else w.theta_local,
+                                None, 0.125, dtype=torch.float64)
+        x = x + a.reshape(-1, w.hidden) @ lw.wo.double().t()
+        y = ln(x, lw.mlp_norm) @ lw.wi.double().t()
+        x = x + (F.gelu(y[:, :w.inter]) * y[:, w.inter:]) @ lw.wo_mlp.double().t()
+    return ln(x, w.final_norm)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D,I", [(64, 64), (128, 192), (768, 1152), (1024, 320), (1088, 64)])
+@pytest.mark.parametrize("lens", [[1], [31], [20, 13], [150, 1, 70], [300, 411], [1000, 30]])
+def test_small_layers(dev, dtype, D, I, lens, monkeypatch):
+    print("small layers", dtype, D, I, lens, flush=True)
+    w = _weights(D, I, dtype, D + I + sum(lens))
+    ids = torch.randint(0, 100, (sum(lens),), generator=torch.Generator().manual_seed(1))
+    cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
+    want, wd = _want(ids, cu, w), w.to(dev)
+    small = mb.modernbert_forward(ids.to(dev), cu.to(dev), max(lens), wd).cpu().double()
+    monkeypatch.setattr(mb, "_SMALL_TOKENS", 0)
+    calls = mb.modernbert_forward(ids.to(dev), cu.to(dev), max(lens), wd).cpu().double()
+    bound = 8.4e-3 if dtype == torch.bfloat16 else 1.05e-3
+    rel = lambda t: float((t - want).norm() / want.norm())
+    assert rel(small) <= bound and rel(calls) <= bound, (rel(small), rel(calls))
+
+
+def test_small_layers_refuse(dev):
+    """Calls that keep the separate kernels: a weight with its own linear, a
+    strided weight, other types, autocast."""
+    w = _weights(128, 64, torch.bfloat16, 3).to(dev)
+    x = torch.zeros(8, 128, dtype=torch.bfloat16, device=dev)
+    cu = torch.tensor([0, 8], dtype=torch.int32, device=dev)
+    assert mb._small_layers(x, cu, w, 2)
+
+    class Own(torch.Tensor):
+        pass
+    keep = w.layers[1].wo
+    for bad in (keep.as_subclass(Own), keep.t(), keep.half()):
+        w.layers[1].wo = bad
+        assert not mb._small_layers(x, cu, w, 2)
+    w.layers[1].wo = keep
+    with torch.autocast("cuda", torch.float16):
+        assert not mb._small_layers(x, cu, w, 2)
+    assert not mb._small_layers(x.float(), cu, w, 2)
+
+
+def test_small_layers_captured(dev):
+    """Capture and several replays, with eager work between them."""
+    w = _weights(128, 64, torch.bfloat16, 4).to(dev)
+    cu = torch.tensor([0, 40, 90], dtype=torch.int32, device=dev)
+    ids = torch.randint(0, 100, (90,), device=dev)
+    call = lambda: mb.modernbert_forward(ids, cu, 50, w)
+    call()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = call()
+    for seed in range(3):
+        ids.copy_(torch.randint(0, 100, (90,), generator=torch.Generator().manual_seed(seed)))
+        graph.replay()
+        got = out.clone()
+        assert torch.equal(got, call())
+        torch.cuda.synchronize()

@@ -391,3 +391,27 @@ def test_packed_weight_cache_with_inference_tensors(monkeypatch):
     wp.packed_weight(w_inf)
     assert len(calls) == 5
     wp.clear_cache()
+
+
+def test_modernbert_layer_argument_errors():
+    """vfk_modernbert_layer_fwd refuses what its kernels do not take, before
+    any launch."""
+    import torch
+
+    from kernels import _lib
+    d = lambda t: _lib.ref(_lib.desc(t))
+    z = lambda *s, dt=torch.bfloat16: torch.zeros(*s, dtype=dt)
+    x, out, pend, n = z(4, 64), z(4, 64), z(4, 64), z(64)
+    wq, wo, wi, wm = z(192, 64), z(64, 64), z(128, 64), z(64, 64)
+    fake = 1 << 20
+
+    def f(x=x, pending=None, an=None, wqkv=wq, mn=n, wi=wi, xo=out, rope=fake, ws=fake, size=1 << 30):
+        _lib.call("vfk_modernbert_layer_fwd", d(x), d(pending), d(an), d(wqkv), d(wo), d(mn), d(wi), d(wm),
+                  1e-5, fake, 1, 4, -1, rope, 256, None, 0.125, ws, size, d(xo), d(pend), None)
+    for bad in (dict(xo=x), dict(wqkv=z(192, 128)), dict(mn=z(65)), dict(mn=n.float()), dict(wi=z(128, 65)),
+                dict(rope=None), dict(ws=None), dict(size=16), dict(xo=z(4, 128)), dict(an=z(32))):
+        with pytest.raises(ValueError):
+            f(**bad)
+    for bad in (dict(x=z(4, 64, dt=torch.float32)), dict(x=z(4, 65)), dict(wi=z(120, 64)), dict(pending=pend)):
+        with pytest.raises(NotImplementedError):
+            f(**bad)

@@ -27,9 +27,7 @@
 // time: a token tile comes from HBM once and from that XCD's L2 after. The K
 // slices of all of a workgroup's tiles form one stream, so the next tile's
 // first slices load while the previous tile's epilogue runs.
-#include "activation.h"
-#include "attn_core.h"
-#include "launch_util.h"
+#include "gemm_small.h"
 
 #include <algorithm>
 
@@ -445,183 +443,25 @@ __global__ __launch_bounds__(256, 1) void gemm_glu_kernel(GluArgs a) {
   __builtin_amdgcn_s_waitcnt(0);  // the repeated last slices
 }
 
-// ---------------------------------------------------------------------------
-// Small token counts: 32 WM tokens x 32 WN features a workgroup (both weight
-// halves), four waves as WM x WN x WK.
-//
-// The 256 x 128 tiles above give ceil(M / 256) ceil(I / 128) workgroups: 9 for
-// one query of 32 tokens and 18 for a document of 500 at I = 1152, each of
-// which walks all of K alone while the rest of the chip idles. Here the same
-// calls give 36 and 144 workgroups, and ST stages keep ST - 1 steps of loads
-// in flight, so that the time is about a memory latency plus the slices:
-// 19.9 -> 5.5 us and 24.3 -> 7.3 us (six stages of 64 x 64, one workgroup a CU
-// instead of two: 8.3 us).
-//
-// A step is WK consecutive 64-wide K slices, one for each of the WK wave
-// groups; wave group wk multiplies slice WK s + wk, and the groups' partial
-// sums meet in LDS at the end. LDS rows are swizzled as above; a stage holds
-// the x rows of all groups, then their weight rows (input half, gate half).
-// ---------------------------------------------------------------------------
-template <int N>
-__device__ inline void step_barrier() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
-}
-
-// 64 lanes' 16 bytes at r + vo + so into the 1 KiB block at lds.
-__device__ inline void lds_load16(rsrc_t r, char* lds, int vo, int so) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)lds, 16, vo, so, 0, 0);
-}
-
-template <typename E, int ACT, int WM, int WN, int WK, int ST>
-__global__ __launch_bounds__(256) void gemm_glu_small_kernel(GluArgs a) {
-  constexpr int TM = 32 * WM, TF = 32 * WN;
-  constexpr int kX = WK * TM * 128, kStage = kX + WK * 2 * TF * 128;
-  constexpr int NX = WK * TM / 32, NW = WK * 2 * TF / 32;  // 8-row loads of a wave per stage
-  constexpr int L = NX + NW;
-  static_assert(WM * WN * WK == 4 && (ST - 2) * L <= 63 && ST >= 2 && ST <= 6, "shape");
-  __shared__ __attribute__((aligned(1024))) char smem[ST * kStage];
-  const int l = threadIdx.x & 63, c = l & 31, h = l >> 5;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int wk = WK == 4 ? w : 0, wm = WK == 4 ? 0 : w / WN, wn = WK == 4 ? 0 : w % WN;
-  // neighbours on one XCD share the operand of which each XCD then needs all;
-  // the larger one is split over the XCDs
-  const int work = xcd_remap(blockIdx.x, gridDim.x);
-  const bool tok_fast = a.M <= 2 * (int64_t)a.I;
-  const int mi = tok_fast ? work % a.mt : work / a.nt;
-  const int ni = tok_fast ? work / a.mt : work % a.nt;
-  const int64_t t0 = (int64_t)mi * TM;
-  const int f0 = ni * TF;
-  const int nk = a.K >> 6, steps = (nk + WK - 1) / WK;
-
-  // rows past the end of x or w read as zeros (features past I of the input
-  // half read gate rows, whose products are not stored); the resources end
-  // with the last row's K values, so that the slices past K of a last step,
-  // which no wave multiplies, stay inside them too
-  const int64_t xrows = a.M - t0 < TM ? a.M - t0 : TM;
-  const rsrc_t xr = uniform_rsrc(a.x + t0 * (a.xs2 >> 1), (int)(xrows - 1) * a.xs2 + 2 * a.K);
-  const rsrc_t wr = uniform_rsrc(a.w, (2 * a.I - 1) * a.ws2 + 2 * a.K);
-  int vx[NX], vw[NW];
-#pragma unroll
-  for (int j = 0; j < NX; ++j) {
-    const int row = 8 * (4 * j + w) + (l >> 3);  // of the stage's x region
-    vx[j] = (row % TM) * a.xs2 + 16 * ((l & 7) ^ swz(row));
-  }
-#pragma unroll
-  for (int j = 0; j < NW; ++j) {
-    const int row = 8 * (4 * j + w) + (l >> 3), r = row % (2 * TF);
-    vw[j] = ((r / TF) * a.I + f0 + r % TF) * a.ws2 + 16 * ((l & 7) ^ swz(row));
-  }
-  auto load = [&](int s, char* st) {
-#pragma unroll
-    for (int j = 0; j < NX; ++j)
-      lds_load16(xr, st + (4 * j + w) * 1024, vx[j], (s * WK + 32 * j / TM) * 128);
-#pragma unroll
-    for (int j = 0; j < NW; ++j)
-      lds_load16(wr, st + kX + (4 * j + w) * 1024, vw[j], (s * WK + 32 * j / (2 * TF)) * 128);
-  };
-#pragma unroll
-  for (int s = 0; s < ST - 1; ++s)
-    if (s < steps) load(s, smem + s * kStage);
-
-  f32x16_t acc[2] = {};
-  int xo[4], wo[4];
-#pragma unroll
-  for (int ds = 0; ds < 4; ++ds) {
-    const int o = 128 * c + 16 * ((2 * ds + h) ^ swz(c));
-    xo[ds] = o + (wk * TM + 32 * wm) * 128;
-    wo[ds] = o + kX + (wk * 2 * TF + 32 * wn) * 128;
-  }
-  int cur = 0, nxt = (ST - 1) * kStage;  // stage offsets of step s and of step s + ST - 1
-  for (int s = 0; s < steps; ++s) {
-    // step s has landed in every wave, and every wave is done with step s - 1
-    switch (min(ST - 2, steps - 1 - s)) {
-      case 0: step_barrier<0>(); break;
-      case 1: step_barrier<(ST > 2 ? 1 : 0) * L>(); break;
-      case 2: step_barrier<(ST > 3 ? 2 : 0) * L>(); break;
-      case 3: step_barrier<(ST > 4 ? 3 : 0) * L>(); break;
-      default: step_barrier<(ST > 5 ? 4 : 0) * L>(); break;
-    }
-    const char* st = smem + cur;
-    u32x4_t xf[4], wf[2][4];
-#pragma unroll
-    for (int ds = 0; ds < 4; ++ds) {
-      xf[ds] = *reinterpret_cast<const u32x4_t*>(st + xo[ds]);
-#pragma unroll
-      for (int g = 0; g < 2; ++g)
-        wf[g][ds] = *reinterpret_cast<const u32x4_t*>(st + wo[ds] + g * TF * 128);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (s + ST - 1 < steps) load(s + ST - 1, smem + nxt);
-    cur = cur == (ST - 1) * kStage ? 0 : cur + kStage;
-    nxt = nxt == (ST - 1) * kStage ? 0 : nxt + kStage;
-    if (WK == 1 || s * WK + wk < nk) {  // uniform in the wave
-#pragma unroll
-      for (int ds = 0; ds < 4; ++ds)
-#pragma unroll
-        for (int g = 0; g < 2; ++g) acc[g] = E::mfma32(wf[g][ds], xf[ds], acc[g]);
-    }
-  }
-  // lane: token t0 + 32 wm + c; feature f0 + 32 wn + 8 j + 4 h + e in register 4 j + e
-  const int64_t t = t0 + 32 * wm + c;
-  uint16_t* orow = a.out + t * a.os;
-  const int fl = f0 + 32 * wn + 4 * h;
-  auto put = [&](int j, const float (&in)[4], const float (&gate)[4]) {
-    const int f = fl + 8 * j;
-    if (t >= a.M || f >= a.I) return;
-    float v[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = act_f<ACT>(in[e]) * gate[e];
-    *reinterpret_cast<u32x2_t*>(orow + f) = u32x2_t{E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
-  };
-  if (WK == 1) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float in[4] = {acc[0][4 * j], acc[0][4 * j + 1], acc[0][4 * j + 2], acc[0][4 * j + 3]};
-      const float gate[4] = {acc[1][4 * j], acc[1][4 * j + 1], acc[1][4 * j + 2], acc[1][4 * j + 3]};
-      put(j, in, gate);
-    }
-    return;
-  }
-  // partial sums of the four K groups through LDS: wave w adds up registers
-  // 4 w .. 4 w + 3 of both halves
-  __syncthreads();  // every wave has read its last operands
-  f32x4_t* red = reinterpret_cast<f32x4_t*>(smem);  // [half][j][wave][lane]
-#pragma unroll
-  for (int g = 0; g < 2; ++g)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      red[((g * 4 + j) * 4 + w) * 64 + l] =
-          f32x4_t{acc[g][4 * j], acc[g][4 * j + 1], acc[g][4 * j + 2], acc[g][4 * j + 3]};
-  __syncthreads();
-  float sum[2][4];
-#pragma unroll
-  for (int g = 0; g < 2; ++g) {
-    f32x4_t x = red[((g * 4 + w) * 4) * 64 + l];
-#pragma unroll
-    for (int u = 1; u < 4; ++u) x += red[((g * 4 + w) * 4 + u) * 64 + l];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) sum[g][e] = x[e];
-  }
-  put(w, sum[0], sum[1]);
-}
-
+// The tiles of gemm_small.h for the arguments of a GLU launch.
 template <typename E, int WM, int WN, int WK, int ST>
-void launch_glu_small(int act, GluArgs& a, hipStream_t st) {
-  a.mt = (int)((a.M + 32 * WM - 1) / (32 * WM));
-  a.nt = (a.I + 32 * WN - 1) / (32 * WN);
-  const int grid = a.mt * a.nt;
+void launch_glu_small(int act, const GluArgs& g, hipStream_t st) {
+  SmallArgs a = {};
+  a.x = g.x; a.w = g.w; a.out = g.out;
+  a.M = g.M; a.K = g.K; a.I = g.I;
+  a.xs2 = g.xs2; a.ws2 = g.ws2; a.os = g.os;
   switch (act) {
     case VFK_ACT_GELU_ERF:
-      gemm_glu_small_kernel<E, VFK_ACT_GELU_ERF, WM, WN, WK, ST><<<grid, 256, 0, st>>>(a);
+      launch_gemm_small<E, VFK_ACT_GELU_ERF, false, 2, WM, WN, WK, ST>(a, st);
       break;
     case VFK_ACT_GELU_TANH:
-      gemm_glu_small_kernel<E, VFK_ACT_GELU_TANH, WM, WN, WK, ST><<<grid, 256, 0, st>>>(a);
+      launch_gemm_small<E, VFK_ACT_GELU_TANH, false, 2, WM, WN, WK, ST>(a, st);
       break;
     case VFK_ACT_SILU:
-      gemm_glu_small_kernel<E, VFK_ACT_SILU, WM, WN, WK, ST><<<grid, 256, 0, st>>>(a);
+      launch_gemm_small<E, VFK_ACT_SILU, false, 2, WM, WN, WK, ST>(a, st);
       break;
     default:
-      gemm_glu_small_kernel<E, VFK_ACT_RELU, WM, WN, WK, ST><<<grid, 256, 0, st>>>(a);
+      launch_gemm_small<E, VFK_ACT_RELU, false, 2, WM, WN, WK, ST>(a, st);
       break;
   }
 }
@@ -642,15 +482,6 @@ void launch_glu(int act, const GluArgs& a, int grid, hipStream_t st) {
       gemm_glu_kernel<E, VFK_ACT_RELU><<<grid, 256, 0, st>>>(a);
       break;
   }
-}
-
-int compute_units() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-      cus < VFK_NUM_XCD)
-    cus = 256;
-  return cus;
 }
 
 // Tiles per XCD and workgroups per XCD (one per CU: the kernel takes all of a
@@ -677,7 +508,7 @@ int persistent_grid(GluArgs& a, int cus) {
 enum GluTile { GLU_32, GLU_64, GLU_256 };
 GluTile glu_tile(const GluArgs& a, int cus) {
   const auto tiles = [&](int64_t m, int64_t f) { return ((a.M + m - 1) / m) * ((a.I + f - 1) / f); };
-  if (tiles(32, 32) <= cus) return GLU_32;
+  if (tiles32_fit(a.M, a.I, cus)) return GLU_32;
   const int64_t rounds = (tiles(kGRows, kGFeat) + cus - 1) / cus;
   if (rounds <= 2 && tiles(64, 64) * 256 <= 1300 * rounds * cus) return GLU_64;
   return GLU_256;

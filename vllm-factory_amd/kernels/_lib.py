@@ -78,6 +78,9 @@ _SIGNATURES = {
     "vfk_rmsnorm_fwd": [_P, _P, _P, _f32, _P, _P, _vp],
     "vfk_glu_fwd": [_i32, _P, _P, _P, _vp],
     "vfk_glu_linear_fwd": [_i32, _P, _P, _P, _vp],
+    "vfk_modernbert_layer_workspace_bytes": [_i32, _i64, _i32, _i32, _i32, _i32],
+    "vfk_modernbert_layer_fwd": [_P, _P, _P, _P, _P, _P, _P, _P, _f32, _vp, _i32, _i32, _i32, _vp, _i32,
+                                 _vp, _f32, _vp, _i64, _P, _P, _vp],
     "vfk_dense_residual_layernorm_fwd": [_P, _P, _P, _P, _P, _P, _f32, _P, _P, _vp],
     "vfk_pack_weight_mfma32": [_P, _P, _vp],
     "vfk_deberta_rel_chunk_major": [_P, _P, _P, _P, _i32, _vp],
@@ -94,6 +97,7 @@ _SIGNATURES = {
 
 _RESTYPES = {"vfk_varlen_attn_workspace_bytes": ctypes.c_int64,
              "vfk_qkv_rope_workspace_bytes": ctypes.c_int64,
+             "vfk_modernbert_layer_workspace_bytes": ctypes.c_int64,
              "vfk_varlen_meta_workspace_bytes": ctypes.c_int64,
              "vfk_gliner_class_workspace_bytes": ctypes.c_int64}
 
