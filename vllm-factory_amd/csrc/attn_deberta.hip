@@ -21,6 +21,8 @@
 
 namespace vfk {
 
+typedef int i32x4_t __attribute__((ext_vector_type(4)));
+
 struct DebArgs {
   const void* q; const void* k; const void* v; void* o;
   int64_t qs[4], ks[4], vs[4], os[4];
@@ -52,6 +54,25 @@ __host__ __device__ inline int deb_index(const DebArgs& a, int d) {
     bk = d;
   }
   return min(max(bk + a.span, 0), 2 * a.span - 1);
+}
+
+// c(d) as deb_index gives it, with the step thresholds in LDS.
+__device__ inline int deb_index_lds(const DebArgs& a, const int16_t* thr, int d) {
+  if (!a.log_bucket) return min(max(d + a.span, 0), 2 * a.span - 1);
+  const int mag = step_eval_lds(a.step, thr, d < 0 ? -d : d);
+  return min(max((d < 0 ? -mag : mag) + a.span, 0), 2 * a.span - 1);
+}
+
+// lut[e] := mul c(dmin + e) for e < n by a 256-thread workgroup. The binary
+// search runs over a copy of the thresholds in thr (LDS, VFK_MAX_THR int16,
+// free for other use after the caller's next barrier): its eight or nine
+// dependent reads are LDS reads of about 0.05 us, where reads of the kernel's
+// arguments are cache reads of several times that, two or three times over
+// per workgroup before its first tile.
+__device__ inline void deb_fill_lut(const DebArgs& a, int16_t* lut, int n, int dmin, int mul, int16_t* thr) {
+  for (int e = threadIdx.x; e < a.step.nthr; e += 256) thr[e] = a.step.thr[e];
+  __syncthreads();
+  for (int e = threadIdx.x; e < n; e += 256) lut[e] = (int16_t)(mul * deb_index_lds(a, thr, dmin + e));
 }
 
 template <typename E>
@@ -88,7 +109,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_kernel(DebArgs a) {
 
   // c(i - j) for d = i - j in [q0 - (kt_end*64 - 1), q0 + 127]
   const int dmin = q0 - (kt_end * kBN - 1);
-  for (int e = t; e < a.lut_len; e += 256) lut[e] = (int16_t)deb_index(a, dmin + e);
+  deb_fill_lut(a, lut, a.lut_len, dmin, 1, reinterpret_cast<int16_t*>(Vt));
 
   const uint16_t* Qp = reinterpret_cast<const uint16_t*>(a.q) + b * a.qs[0] + h * a.qs[1];
   const uint16_t* Kp = reinterpret_cast<const uint16_t*>(a.k) + b * a.ks[0] + h * a.ks[1];
@@ -152,7 +173,13 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_kernel(DebArgs a) {
 // pos_key columns of a query row, and the 128 query rows of the workgroup
 // meet at most 128 consecutive pos_query columns of a key row. Windows start
 // on an 8-column boundary (kPkW = 64 + 8, kPqW = 128 + 8) and are clamped
-// into [0, 2S). The scores then read their biases from LDS.
+// into [0, 2S). The scores then read their biases from LDS. A wave issues its
+// instructions alone or beside one other, so their number per score counts:
+// rows' offsets are read four at a time, in bytes, and where c(d) = d + span
+// for the whole tile the column is an immediate and the table is not read (8 x
+// 12 x 371, bf16: 41.3 -> 37.2 us, of which 1 us from filling the table
+// through LDS thresholds). Fetching the windows one tile ahead measured slower
+// (43.3 against 41.4 us: 40 more registers live through the products).
 constexpr int kPkW = kBN + 8;        // staged pos_key columns per query row
 constexpr int kPqW = kBM + 8;        // staged pos_query columns per key row
 constexpr int kPkChunks = kPkW / 8;  // 16-byte chunks per staged row
@@ -170,9 +197,9 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
   uint16_t* Vt = Ks + kKsElems;
   uint16_t* PKs = Vt + kVtElems;                            // [kBM][kPkW]
   uint16_t* PQs = PKs + kBM * kPkW;                         // [kBN][kPqW]
-  int* pko = reinterpret_cast<int*>(PQs + kBN * kPqW);      // [kBM] row * kPkW - window start
-  int* pqo = pko + kBM;                                     // [kBN] row * kPqW - window start
-  int16_t* lut = reinterpret_cast<int16_t*>(pqo + kBN);    // c(i - j)
+  int* pko = reinterpret_cast<int*>(PQs + kBN * kPqW);      // [kBM] bytes: row * kPkW - window start
+  int* pqo = pko + kBM;                                     // [kBN] bytes: row * kPqW - window start
+  int16_t* lut = reinterpret_cast<int16_t*>(pqo + kBN);    // 2 c(i - j)
 
   const int nqt = (a.M + kBM - 1) / kBM;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
@@ -199,7 +226,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
   }
 
   const int dmin = q0 - (kt_end * kBN - 1);
-  for (int e = t; e < a.lut_len; e += 256) lut[e] = (int16_t)deb_index(a, dmin + e);
+  deb_fill_lut(a, lut, a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vt));
 
   const uint16_t* Qp = reinterpret_cast<const uint16_t*>(a.q) + b * a.qs[0] + h * a.qs[1];
   const uint16_t* Kp = reinterpret_cast<const uint16_t*>(a.k) + b * a.ks[0] + h * a.ks[1];
@@ -228,7 +255,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
     for (int u = 0; u < 5 && PK; ++u) {
       const int c = min(t + 256 * u, kBM * kPkChunks - 1);
       const int r = c / kPkChunks, j = c - r * kPkChunks;
-      const int cmin = lut[q0 + r - key0 - (kBN - 1) - dmin];
+      const int cmin = lut[q0 + r - key0 - (kBN - 1) - dmin] >> 1;
       const int start = min(cmin & ~7, span2 - kPkW);
       pkv[u] = *reinterpret_cast<const u32x4_t*>(PKp + (int64_t)min(q0 + r, a.M - 1) * a.pks[2] +
                                                  start + 8 * j);
@@ -237,19 +264,19 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
     for (int u = 0; u < 5 && PQ; ++u) {
       const int c = min(t + 256 * u, kBN * kPqChunks - 1);
       const int r = c / kPqChunks, j = c - r * kPqChunks;
-      const int cmin = lut[q0 - key0 - r - dmin];
+      const int cmin = lut[q0 - key0 - r - dmin] >> 1;
       const int start = min(cmin & ~7, span2 - kPqW);
       pqv[u] = *reinterpret_cast<const u32x4_t*>(PQp + (int64_t)min(key0 + r, a.N - 1) * a.pqs[2] +
                                                  start + 8 * j);
     }
     kv_store(st, Ks, Vt);
     if (PK && t < kBM) {
-      const int cmin = lut[q0 + t - key0 - (kBN - 1) - dmin];
-      pko[t] = t * kPkW - min(cmin & ~7, span2 - kPkW);
+      const int cmin = lut[q0 + t - key0 - (kBN - 1) - dmin] >> 1;
+      pko[t] = 2 * (t * kPkW - min(cmin & ~7, span2 - kPkW));
     } else if (PQ && t >= kBM && t < kBM + kBN) {
       const int r = t - kBM;
-      const int cmin = lut[q0 - key0 - r - dmin];
-      pqo[r] = r * kPqW - min(cmin & ~7, span2 - kPqW);
+      const int cmin = lut[q0 - key0 - r - dmin] >> 1;
+      pqo[r] = 2 * (r * kPqW - min(cmin & ~7, span2 - kPqW));
     }
     __syncthreads();
     if (kt + 1 < kt_end) kv_load(st, Kp, a.ks[2], Vp, a.vs[2], (kt + 1) * kBN, kend);
@@ -270,19 +297,44 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
     }
     __syncthreads();
 
-    const int16_t* lp = lut + (lut_lane - key0);
-    const uint16_t* pkr = PKs + (PK ? pko[prow] : 0);
-    map_scores(s0, s1, [&](int e, float v) {
-      const int xk = x_key(e, 0);  // key - key0 - 4*hl
-      const int kr = xk + 4 * hl;
-      const int key = key0 + kr;
-      const int c = lp[-xk];
-      float bias = 0.f;  // summed as the per-score gather does: bit-equal
-      if (PK) bias += E::to_f32(pkr[c]);
-      if (PQ) bias += E::to_f32(PQs[pqo[kr] + c]);
-      v += bias;
-      return (key >= kend || (a.causal && key > qrow + (a.N - a.M))) ? -INFINITY : v;
-    });
+    // byte offset of column 0 in the lane's staged pos_key row; pqo holds that
+    // of its keys' pos_query rows (runs of four)
+    const int pk0 = PK ? pko[prow] : 0;
+    // adds the terms of 16 scores (the tile's keys 32 hf ..): the lane columns
+    // from col(e) in bytes; their sum is formed first, as the per-score gather does
+    auto add_terms = [&](f32x16_t& sv, int hf, auto col) {
+      i32x4_t pq0[4];
+#pragma unroll
+      for (int j = 0; j < 4 && PQ; ++j)
+        pq0[j] = *reinterpret_cast<const i32x4_t*>(pqo + 32 * hf + 8 * j + 4 * hl);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int c2 = col(16 * hf + e);
+        const float pk = PK ? E::to_f32(lds_at<uint16_t>(PKs, pk0 + c2)) : 0.f;
+        const float pq = PQ ? E::to_f32(lds_at<uint16_t>(PQs, pq0[e >> 2][e & 3] + c2)) : 0.f;
+        sv[e] += PK && PQ ? pk + pq : PK ? pk : pq;
+      }
+    };
+    // where every distance of the wave's rows has c(d) = d + span, the column
+    // is a lane value plus an immediate
+    const int qw0 = q0 + w * 32;
+    if (__builtin_amdgcn_readfirstlane((int)(qw0 - key0 - (kBN - 1) >= a.lin_lo && qw0 + 31 - key0 <= a.lin_hi))) {
+      const int c2 = 2 * (qrow - 4 * hl - key0 + a.span);
+      auto col = [&](int e) { return c2 - 2 * x_key(e, 0); };
+      add_terms(s0, 0, col);
+      add_terms(s1, 1, col);
+    } else {
+      const int16_t* lp = lut + (lut_lane - key0);
+      auto col = [&](int e) { return (int)lp[-x_key(e, 0)]; };
+      add_terms(s0, 0, col);
+      add_terms(s1, 1, col);
+    }
+    if (a.causal || key0 + kBN > kend) {  // some row does not see some key of the tile
+      map_scores(s0, s1, [&](int e, float v) {
+        const int key = key0 + x_key(e, hl);
+        return (key >= kend || (a.causal && key > qrow + (a.N - a.M))) ? -INFINITY : v;
+      });
+    }
     u32x4_t p[4];
     softmax_tile<E>(s0, s1, a.c2, m, l, o0, o1, p);
     pv_tile<E>(Vt, p, o0, o1);
@@ -387,11 +439,8 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_f32_kernel(DebArgs a, D
     pol.hi = min(max(f.q0 + kF32Rows - 1, -x.sat), x.sat);
     for (int e = t; e < a.step.nthr; e += 256) thr[e] = a.step.thr[e];
     __syncthreads();
-    for (int e = t; e <= pol.hi - pol.lo; e += 256) {
-      const int d = pol.lo + e;
-      const int mag = step_eval_lds(a.step, thr, d < 0 ? -d : d);
-      lutc[e] = (int16_t)min(max((d < 0 ? -mag : mag) + a.span, 0), 2 * a.span - 1);
-    }
+    for (int e = t; e <= pol.hi - pol.lo; e += 256)
+      lutc[e] = (int16_t)deb_index_lds(a, thr, pol.lo + e);
     __syncthreads();
   }
   pol.qrow = f.q0 + (t & 15);
@@ -551,7 +600,7 @@ __global__ __launch_bounds__(256, 2) void deberta_fused_kernel(DebArgs a) {
   }
   const int kt_end = (len + kBN - 1) / kBN;
   const int dmin = q0 - (kt_end * kBN - 1);
-  for (int e = t; e < a.lut_len; e += 256) lut[e] = (int16_t)(2 * deb_index(a, dmin + e));
+  deb_fill_lut(a, lut, a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vs));
 
   const uint16_t* Qp = reinterpret_cast<const uint16_t*>(a.q) + qb + h * a.qs[1];
   TileSrc ksrc, vsrc;
