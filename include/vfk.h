@@ -510,6 +510,18 @@ int vfk_glu_fwd(int32_t act, const vfk_tensor* a, const vfk_tensor* b,
 int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_tensor* w,
                        vfk_tensor* out, void* stream);
 
+/* vfk_varlen_attn_fwd with RoPE for few queries: the keys are rotated where
+ * they are used, without a pre-pass and its workspace, and the waves of a
+ * workgroup split them. Same arguments and results to rounding; bf16 / fp16,
+ * rope table required. vfk_varlen_attn_direct: 1 where this form is the
+ * faster one. */
+int vfk_varlen_attn_direct(int32_t dtype, int32_t num_heads, int32_t num_seqs, int32_t max_seqlen);
+int vfk_varlen_attn_direct_fwd(const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,
+                               const int32_t* cu_seqlens, int32_t num_seqs, int32_t max_seqlen,
+                               int32_t window, const float* rope_cos_sin, int32_t rope_positions,
+                               const uint8_t* key_valid, float softmax_scale, vfk_tensor* out,
+                               void* stream);
+
 /* One ModernBERT layer over packed sequences (models/modernbert/
  * modernbert_encoder.py:289-352), for few tokens: all of its kernels are
  * enqueued by one call, the products run on 32 x 32 and 64 x 128 tiles.

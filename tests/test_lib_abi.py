@@ -415,3 +415,28 @@ def test_modernbert_layer_argument_errors():
     for bad in (dict(x=z(4, 64, dt=torch.float32)), dict(x=z(4, 65)), dict(wi=z(120, 64)), dict(pending=pend)):
         with pytest.raises(NotImplementedError):
             f(**bad)
+
+
+def test_varlen_direct_rule_and_errors():
+    """The rule is a function of sizes and type alone; the form refuses what
+    the one with a workspace refuses."""
+    import torch
+
+    from kernels import _lib
+    rule = _lib.load().vfk_varlen_attn_direct
+    assert rule(_lib.BF16, 12, 1, 300) == 1 and rule(_lib.F16, 12, 16, 128) == 1
+    assert rule(_lib.BF16, 12, 2, 700) == 0 and rule(_lib.BF16, 12, 17, 128) == 0
+    assert rule(_lib.F32, 12, 1, 32) == 0 and rule(_lib.BF16, 1, 1, 1 << 24) == 0
+    d = lambda t: _lib.ref(_lib.desc(t))
+    fake = 1 << 20
+    q = torch.zeros(8, 2, 64, dtype=torch.bfloat16)
+
+    def f(q=q, cu=fake, window=-1, rope=fake, npos=256, scale=0.125, out=q):
+        _lib.call("vfk_varlen_attn_direct_fwd", d(q), d(q), d(q), cu, 1, 8, window, rope, npos, None, scale,
+                  d(out), None)
+    for bad in (dict(cu=None), dict(rope=None), dict(npos=4), dict(out=torch.zeros(8, 3, 64, dtype=q.dtype))):
+        with pytest.raises(ValueError):
+            f(**bad)
+    for bad in (dict(scale=0.0), dict(q=q.float(), out=q.float())):
+        with pytest.raises(NotImplementedError):
+            f(**bad)

@@ -481,6 +481,156 @@ __global__ __launch_bounds__(256, 4) void varlen_fwd_kernel(VarlenArgs a) {
                   a.os[0], n, nfull);
 }
 
+// Few queries: one workgroup per 32 query rows of one (sequence, head), whose
+// four waves split the keys. The workgroups above own 128 rows and walk all
+// their keys in one chain, after a launch that rotates K: 11 tiles of about
+// 1.4 us for a document of 700 tokens on 144 workgroups. Here wave w takes the
+// 64-key tiles w, w + 4, ... by itself: its K rows go from global memory
+// straight into the operand registers, where they are rotated (the same
+// arithmetic and the same one rounding as the pre-pass), its V tile through
+// its own LDS, with no barrier before the waves' outputs are merged. Each
+// workgroup rotates the K rows it reads, so that a row is rotated once per 32
+// queries instead of once: taken while the 128-row workgroups leave the chip
+// idle (vfk_varlen_attn_direct).
+constexpr int kDirRows = 32;
+constexpr int kDirPad = 68;  // floats per merged output row
+// Largest product of 128-row items (sequences x heads x query tiles of the
+// longest) and query tiles of a call that takes it, 192: with the number of
+// items the workgroups of 128 rows fill the chip, with the length each row's
+// keys are rotated by more workgroups. Two layers (one global, one local) of
+// 12 heads, us, this form against the other: 1 x 32 tokens 22 against 33, 1 x
+// 300 23 against 33, 8 x 40 23 against 38, 16 x 120 30 against 35; past the
+// line 8 x 250 39 against 36, 2 x 700 50 against 35, 4 x 1100 137 against 55.
+constexpr int kDirectMaxWork = 192;
+
+// The wave's 64 V rows from key0 on into its own LDS tile.
+__device__ inline void wave_tile_load(rsrc_t r, int rs2, int key0, uint16_t* tile) {
+  const int p = threadIdx.x & 63;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int row = 8 * j + (p >> 3);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)(tile + j * 512), 16,
+                                             row * rs2 + 16 * ((p & 7) ^ swz(row)), key0 * rs2, 0, 0);
+  }
+}
+
+template <typename E>
+__global__ __launch_bounds__(256, 2) void varlen_direct_kernel(VarlenArgs a) {
+  // the waves' V tiles in the loop, their outputs after it
+  __shared__ __align__(16) unsigned char smem[4 * kDirRows * kDirPad * 4];
+  __shared__ float ms[4][kDirRows], ls[4][kDirRows];
+  const int work = xcd_remap(blockIdx.x, gridDim.x);
+  const int qt = work % a.nqt;
+  const int h = (work / a.nqt) % a.H;
+  const int s = work / (a.nqt * a.H);
+  const int t = threadIdx.x, lane = t & 63, c = lane & 31, hl = lane >> 5;
+  const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int tok0 = a.cu[s], nfull = a.cu[s + 1] - tok0, n = min(nfull, a.maxlen);
+  uint16_t* ob = reinterpret_cast<uint16_t*>(a.o) + (int64_t)tok0 * a.os[0] + h * a.os[1];
+  if (qt == a.nqt - 1 && nfull > n) zero_rows_d64(ob, a.os[0], n, nfull);
+  const int q0 = qt * kDirRows;
+  if (q0 >= n) return;  // whole workgroup: uniform exit
+  const int qrow = q0 + c, window = a.window;
+  const uint16_t* Kp = reinterpret_cast<const uint16_t*>(a.k) + (int64_t)tok0 * a.ks[0] + h * a.ks[1];
+  const uint16_t* Vp = reinterpret_cast<const uint16_t*>(a.v) + (int64_t)tok0 * a.vs[0] + h * a.vs[1];
+  const int rs2 = (int)a.vs[0] * 2;
+  const rsrc_t vr = uniform_rsrc(Vp, n * rs2);  // rows past n read as zeros
+  uint16_t* Vt = reinterpret_cast<uint16_t*>(smem) + w * kTileElems;
+  RopeQ rq;
+  rope_q_fetch(rq, a.rope + (int64_t)min(qrow, n - 1) * 64);
+  u32x4_t qf[4];
+  load_q(qf, reinterpret_cast<const uint16_t*>(a.q) + (int64_t)(tok0 + min(qrow, n - 1)) * a.qs[0] + h * a.qs[1],
+         qrow < n);
+  rope_q_apply<E>(qf, rq);
+  VOff vo;
+  v_offsets(vo);
+  float m = -INFINITY;
+  RowSumDot<E> l;
+  f32x16_t o0 = {}, o1 = {};
+  const int kt_begin = window >= 0 ? max(0, q0 - window) / kBN : 0;
+  const int kt_end = ((window >= 0 ? min(n, q0 + kDirRows + window) : n) + kBN - 1) / kBN;
+  for (int kt = kt_begin + w; kt < kt_end; kt += 4) {
+    const int key0 = kt * kBN;
+    wave_tile_load(vr, rs2, key0, Vt);
+    u32x4_t k[2][4];
+    RopeK rk[2][2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      const int j = min(key0 + 32 * kb + c, n - 1);
+      const uint16_t* row = Kp + (int64_t)j * a.ks[0] + 8 * hl;
+#pragma unroll
+      for (int ds = 0; ds < 4; ++ds) k[kb][ds] = *reinterpret_cast<const u32x4_t*>(row + 16 * ds);
+#pragma unroll
+      for (int dl = 0; dl < 2; ++dl) rope_k_fetch(rk[kb][dl], a.rope, j, 2 * dl + hl);
+    }
+    // keys that exist and are not hidden, one per lane
+    const unsigned long long vm = __builtin_amdgcn_ballot_w64(
+        key0 + lane < n && (!a.key_valid || a.key_valid[tok0 + min(key0 + lane, n - 1)] != 0));
+    f32x16_t s0 = {}, s1 = {};
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+#pragma unroll
+      for (int dl = 0; dl < 2; ++dl) {
+        const u32x4_t lo = rope_k_half<E>(k[kb][dl], k[kb][dl + 2], rk[kb][dl], -1.f, a.c2);
+        k[kb][dl + 2] = rope_k_half<E>(k[kb][dl + 2], k[kb][dl], rk[kb][dl], 1.f, a.c2);
+        k[kb][dl] = lo;
+      }
+    }
+#pragma unroll
+    for (int ds = 0; ds < 4; ++ds) {
+      s0 = E::mfma32(k[0][ds], qf[ds], s0);
+      s1 = E::mfma32(k[1][ds], qf[ds], s1);
+    }
+    const bool cut = window >= 0 && (q0 + kDirRows - 1 - key0 > window || key0 + kBN - 1 - q0 > window);
+    if (vm != ~0ull || cut) {  // uniform
+      const uint32_t lo = (uint32_t)(vm >> (4 * hl)), hi = (uint32_t)(vm >> (32 + 4 * hl));
+      const int d0 = qrow - key0 - 4 * hl;  // qrow - key of element e is d0 - x_key(e, 0)
+      const int win = window >= 0 ? window : 0x3fffffff;
+      map_scores(s0, s1, [&](int e, float v) {
+        const int xk = x_key(e, 0), d = d0 - xk;
+        const bool on = ((xk < 32 ? lo >> xk : hi >> (xk - 32)) & 1u) != 0u;
+        return on && d <= win && d >= -win ? v : -INFINITY;
+      });
+    }
+    u32x4_t p[4];
+    softmax_tile<E>(s0, s1, 1.f, m, l, o0, o1, p);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the V tile is in LDS
+    pv_tile_sw<E>(Vt, vo, p, o0, o1);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // and read, before the next one
+  }
+  const float lt = l.total();
+  if (hl == 0) {
+    ms[w][c] = m;
+    ls[w][c] = lt;
+  }
+  __syncthreads();  // every wave is done with its V tile
+  float* om = reinterpret_cast<float*>(smem) + (w * kDirRows + c) * kDirPad + 4 * hl;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    *reinterpret_cast<f32x4_t*>(om + 8 * j) = f32x4_t{o0[4 * j], o0[4 * j + 1], o0[4 * j + 2], o0[4 * j + 3]};
+    *reinterpret_cast<f32x4_t*>(om + 32 + 8 * j) = f32x4_t{o1[4 * j], o1[4 * j + 1], o1[4 * j + 2], o1[4 * j + 3]};
+  }
+  __syncthreads();
+  const int r = t >> 3, d = 8 * (t & 7);  // eight threads a row
+  if (q0 + r >= n) return;
+  float mm = ms[0][r];
+#pragma unroll
+  for (int u = 1; u < 4; ++u) mm = fmax_ieee(mm, ms[u][r]);
+  float lsum = 0.f, x[8] = {};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const float f = ms[u][r] == -INFINITY ? 0.f : fast_exp2(ms[u][r] - mm);
+    const float* src = reinterpret_cast<const float*>(smem) + (u * kDirRows + r) * kDirPad + d;
+    lsum = __builtin_fmaf(f, ls[u][r], lsum);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = __builtin_fmaf(f, src[e], x[e]);
+  }
+  const float inv = lsum > 0.f ? 1.0f / lsum : 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] *= inv;
+  *reinterpret_cast<u32x4_t*>(ob + (int64_t)(q0 + r) * a.os[0] + d) = pack8<E>(x);
+}
+
 // fp32: one thread per query row, exact fp32 arithmetic, accurate sin/cos.
 __global__ __launch_bounds__(64) void varlen_fwd_f32_kernel(VarlenArgs a) {
   __shared__ float Kt[64][kHD + 1];
@@ -610,13 +760,12 @@ extern "C" int64_t vfk_varlen_attn_workspace_bytes(int32_t dtype, int64_t total_
   return kr_bytes(total_tokens, num_heads) + (int64_t)num_heads * num_seqs * nkt * 16;
 }
 
-extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
-                                   const vfk_tensor* v, const int32_t* cu_seqlens,
-                                   int32_t num_seqs, int32_t max_seqlen,
-                                   int32_t window, const float* rope_cos_sin,
-                                   int32_t rope_positions, const uint8_t* key_valid,
-                                   float softmax_scale, void* workspace,
-                                   int64_t workspace_bytes, vfk_tensor* out, void* stream) {
+// Checks of the packed attention call shared by its two forms; fills a.
+// Returns VFK_OK with a.nseq = 0 where there is nothing to do.
+static int varlen_setup(VarlenArgs& a, const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,
+                        const int32_t* cu_seqlens, int32_t num_seqs, int32_t max_seqlen, int32_t window,
+                        const float* rope_cos_sin, int32_t rope_positions, const uint8_t* key_valid,
+                        float softmax_scale, vfk_tensor* out) {
   int rc = check_tensor(q, "q", 3);
   if (rc) return rc;
   const int dt = q->dtype;
@@ -629,14 +778,14 @@ extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
     return set_error(VFK_ERR_INVALID, "num_seqs/max_seqlen must be >= 0");
   if (T >= (1ll << 31) || H > 4096 || max_seqlen > (1 << 24))
     return set_error(VFK_ERR_UNSUPPORTED, "vfk_varlen_attn_fwd: sizes too large");
+  a.nseq = 0;
   if (num_seqs == 0 || max_seqlen == 0 || H == 0) return VFK_OK;
-  VarlenArgs a = {};
   a.q = q->data; a.k = k->data; a.v = v->data; a.o = out->data;
   for (int i = 0; i < 2; ++i) {
     a.qs[i] = q->stride[i]; a.ks[i] = k->stride[i];
     a.vs[i] = v->stride[i]; a.os[i] = out->stride[i];
   }
-  a.cu = cu_seqlens; a.nseq = num_seqs; a.H = (int)H; a.T = T; a.maxlen = max_seqlen;
+  a.cu = cu_seqlens; a.H = (int)H; a.T = T; a.maxlen = max_seqlen;
   a.window = window < 0 ? -1 : window;
   if (!(softmax_scale > 0.f) || !isfinite(softmax_scale))
     return set_error(VFK_ERR_UNSUPPORTED, "vfk_varlen_attn_fwd: softmax_scale must be > 0");
@@ -650,6 +799,23 @@ extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
       return set_error(VFK_ERR_INVALID, "rope table must be 16-byte aligned");
   }
   a.rope = rope_cos_sin;
+  a.nseq = num_seqs;
+  return VFK_OK;
+}
+
+extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
+                                   const vfk_tensor* v, const int32_t* cu_seqlens,
+                                   int32_t num_seqs, int32_t max_seqlen,
+                                   int32_t window, const float* rope_cos_sin,
+                                   int32_t rope_positions, const uint8_t* key_valid,
+                                   float softmax_scale, void* workspace,
+                                   int64_t workspace_bytes, vfk_tensor* out, void* stream) {
+  VarlenArgs a = {};
+  int rc = varlen_setup(a, q, k, v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin, rope_positions,
+                        key_valid, softmax_scale, out);
+  if (rc || a.nseq == 0) return rc;
+  const int dt = q->dtype;
+  const int64_t T = a.T, H = a.H;
   hipStream_t st = (hipStream_t)stream;
   if (dt == VFK_F32) {
     a.nqt = ceil_div(max_seqlen, 128);
@@ -692,6 +858,43 @@ extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
 #undef VFK_PACK
   }
   return launch_varlen(a, dt, rope, max_seqlen, st, "vfk_varlen_attn_fwd");
+}
+
+extern "C" int vfk_varlen_attn_direct(int32_t dtype, int32_t num_heads, int32_t num_seqs, int32_t max_seqlen) {
+  if (dtype != VFK_BF16 && dtype != VFK_F16) return 0;
+  const int64_t nqt = ceil_div(max_seqlen, kBM);
+  return nqt <= kDirectMaxWork && (int64_t)num_heads * num_seqs * nqt * nqt <= kDirectMaxWork ? 1 : 0;
+}
+
+extern "C" int vfk_varlen_attn_direct_fwd(const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,
+                                          const int32_t* cu_seqlens, int32_t num_seqs, int32_t max_seqlen,
+                                          int32_t window, const float* rope_cos_sin, int32_t rope_positions,
+                                          const uint8_t* key_valid, float softmax_scale, vfk_tensor* out,
+                                          void* stream) {
+  const char* nm = "vfk_varlen_attn_direct_fwd";
+  VarlenArgs a = {};
+  int rc = varlen_setup(a, q, k, v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin, rope_positions,
+                        key_valid, softmax_scale, out);
+  if (rc) return rc;
+  if (q->dtype == VFK_F32) return set_error(VFK_ERR_UNSUPPORTED, "%s: bf16 or fp16 only", nm);
+  if (!rope_cos_sin) return set_error(VFK_ERR_INVALID, "%s: rope table missing", nm);
+  if (a.nseq == 0) return VFK_OK;
+  if (a.window >= max_seqlen) a.window = -1;  // window covers every pair
+  // as the other form, so that a call does not depend on the one it takes
+  if (a.window > kPenOff - kBM)
+    return set_error(VFK_ERR_UNSUPPORTED, "%s: window %d > %d", nm, a.window, kPenOff - kBM);
+  const int64_t span = (int64_t)max_seqlen * 2;  // buffer resource of the V rows
+  if (span * a.ks[0] >= (1ll << 31) || span * a.vs[0] >= (1ll << 31))
+    return set_error(VFK_ERR_UNSUPPORTED, "%s: max_seqlen x row stride too large", nm);
+  a.nqt = ceil_div(max_seqlen, kDirRows);
+  const int64_t blocks = (int64_t)a.nqt * a.H * num_seqs;
+  if (blocks >= (1ll << 31)) return set_error(VFK_ERR_UNSUPPORTED, "%s: grid too large", nm);
+  hipStream_t st = (hipStream_t)stream;
+  if (q->dtype == VFK_BF16)
+    hipLaunchKernelGGL(varlen_direct_kernel<BF16>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(varlen_direct_kernel<F16>, dim3((unsigned)blocks), dim3(256), 0, st, a);
+  return launch_status(nm);
 }
 
 // Attention over K already rotated, scaled by c2 and laid out head-major by

@@ -8,8 +8,8 @@
 // their 32 x 32 tiles fit the chip, the residual add and the LayerNorm in
 // front of Wqkv and Wi are done by those products themselves, so that a layer
 // is six launches instead of eight. 22 layers of width 768 with the embedding
-// and the head, one query of 32 tokens: 2.81 ms as separate calls, 0.77 as one
-// call a layer (kernels 1.05 -> 0.80 ms, host 2.8 -> 0.67).
+// and the head, one query of 32 tokens: 2.81 ms as separate calls, 0.72 as one
+// call a layer (kernels 1.05 -> 0.74 ms, host 2.8 -> 0.57).
 #include <math.h>
 
 #include "gemm_small.h"
@@ -186,10 +186,18 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
   const vfk_tensor q = heads3(qkv, dt, M, 3 * D, H), k = heads3(qkv + D, dt, M, 3 * D, H),
                    v = heads3(qkv + 2 * D, dt, M, 3 * D, H);
   vfk_tensor att = heads3(ws + buf.att, dt, M, D, H);
-  if ((rc = vfk_varlen_attn_fwd(&q, &k, &v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin,
+  // the split keys are summed in another order than one chain sums them: as
+  // with the split K of the products, only where those split K too, so that a
+  // sequence of more tokens gives the same bits alone and in a large pack
+  if (tiles32_fit(M, 3 * D, cus) && vfk_varlen_attn_direct(dt, (int32_t)H, num_seqs, max_seqlen)) {
+    if ((rc = vfk_varlen_attn_direct_fwd(&q, &k, &v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin,
+                                         rope_positions, key_valid, softmax_scale, &att, stream)))
+      return rc;
+  } else if ((rc = vfk_varlen_attn_fwd(&q, &k, &v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin,
                                 rope_positions, key_valid, softmax_scale, ws + buf.attn,
-                                buf.total - buf.attn, &att, stream)))
+                                buf.total - buf.attn, &att, stream))) {
     return rc;
+  }
   const bool narrow = tiles32_fit(M, D, cus);
   {
     const SmallArgs a = small_args(att.data, D, wo, o.data, D, M, D);

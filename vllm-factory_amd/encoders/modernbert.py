@@ -120,7 +120,7 @@ def _dense_ln_fusable(wo: torch.Tensor) -> bool:
 
 # Token count up to which a layer runs as one call on the library's own small
 # tiles (vfk_modernbert_layer_fwd) instead of seven calls. 22 layers of width
-# 768, ms, one call a layer against seven: 32 tokens 0.77 against 2.9, 300 1.07
+# 768, ms, one call a layer against seven: 32 tokens 0.72 against 2.9, 300 1.07
 # against 2.8, 1262 1.44 against 2.9, 3147 2.16 against 2.9, 3935 2.5 against
 # 2.8 (seven calls are bound by the host there), 5549 3.2 against 3.0, 13090
 # 5.7 against 5.0 (the large tiles of the library products win).

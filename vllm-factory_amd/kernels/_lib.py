@@ -56,6 +56,8 @@ _SIGNATURES = {
                                      _vp],
     "vfk_varlen_attn_fwd": [_P, _P, _P, _vp, _i32, _i32, _i32, _vp, _i32, _vp, _f32, _vp, _i64,
                             _P, _vp],
+    "vfk_varlen_attn_direct": [_i32, _i32, _i32, _i32],
+    "vfk_varlen_attn_direct_fwd": [_P, _P, _P, _vp, _i32, _i32, _i32, _vp, _i32, _vp, _f32, _P, _vp],
     "vfk_varlen_attn_workspace_bytes": [_i32, _i64, _i32, _i32, _i32, _i32],
     "vfk_rope_table": [_f32, _i32, _vp, _vp],
     "vfk_varlen_meta": [_vp, _i32, _i64, _i32, _vp, _vp, _vp, _i64, _vp],

@@ -79,6 +79,15 @@ def varlen_rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if rope:
         tab = rope_table(rope_theta, int(max_seqlen), dev)
         tab_ptr, tab_n = tab.data_ptr(), tab.shape[0]
+        if _lib.load().vfk_varlen_attn_direct(_lib.dtype_code(q.dtype), q.shape[1], cu_seqlens.numel() - 1,
+                                              int(max_seqlen)):
+            # few queries: keys rotated in the attention kernel, no workspace
+            _lib.on_device(
+                "vfk_varlen_attn_direct_fwd", dev,
+                _lib.ref(_lib.desc(qq)), _lib.ref(_lib.desc(kk)), _lib.ref(_lib.desc(vv)),
+                cu_seqlens.data_ptr(), int(cu_seqlens.numel() - 1), int(max_seqlen),
+                int(window), tab_ptr, int(tab_n), kv_ptr, float(scale), _lib.ref(_lib.desc(out)))
+            return out
     ws_bytes = int(_lib.load().vfk_varlen_attn_workspace_bytes(
         _lib.dtype_code(q.dtype), int(q.shape[0]), int(q.shape[1]), int(rope),
         int(cu_seqlens.numel() - 1), int(max_seqlen)))
