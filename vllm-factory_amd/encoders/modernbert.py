@@ -9,6 +9,8 @@ rounds the GLU output once where the reference rounds the projection first.
 Wqkv and the rotary step of k run as one kernel (qkv_rope_projection), which
 rotates the fp32 projection sums of k and rounds once; the attention then
 reads that rotated k (varlen_rope_attention_krot) with no separate k pass.
+Up to _SMALL_TOKENS tokens a layer is one call (vfk_modernbert_layer_fwd) that
+enqueues the library's own products, norms and attention.
 Global layers (layer_id % 3 == 0) attend inside each sequence with RoPE theta
 160000, local layers within |i - j| <= 64 with theta 10000; tokens with id
 50284 are hidden as keys (:456-460).

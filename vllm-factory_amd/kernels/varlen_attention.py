@@ -12,7 +12,8 @@ the same attention per sequence from cu_seqlens:
     (ModernBERT local layers use w = local_attention // 2 = 64);
   * rope_theta > 0: q and k are rotated with the HF ModernBertRotaryEmbedding
     frequencies (non-interleaved halves): k once by a pre-pass into a
-    workspace, q inside the attention kernel (inputs are never written);
+    workspace, or, where the call has few queries, inside the attention kernel
+    as q always is (inputs are never written);
   * key_valid[t] == 0 hides key t (the reference's token-id 50284 mask).
 
 Rows that see no key at all are returned as zeros.
