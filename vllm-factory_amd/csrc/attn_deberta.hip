@@ -63,7 +63,7 @@ __device__ inline int deb_index_lds(const DebArgs& a, const int16_t* thr, int d)
   return min(max((d < 0 ? -mag : mag) + a.span, 0), 2 * a.span - 1);
 }
 
-// lut[e] := mul c(dmin + e) for e < n by a 256-thread workgroup. The binary
+// lut[e] := mul c(dmin + e) (its low 16 bits) for e < n by a 256-thread workgroup. The binary
 // search runs over a copy of the thresholds in thr (LDS, VFK_MAX_THR int16,
 // free for other use after the caller's next barrier): its eight or nine
 // dependent reads are LDS reads of about 0.05 us, where reads of the kernel's
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
   uint16_t* PQs = PKs + kBM * kPkW;                         // [kBN][kPqW]
   int* pko = reinterpret_cast<int*>(PQs + kBN * kPqW);      // [kBM] bytes: row * kPkW - window start
   int* pqo = pko + kBM;                                     // [kBN] bytes: row * kPqW - window start
-  int16_t* lut = reinterpret_cast<int16_t*>(pqo + kBN);    // 2 c(i - j)
+  uint16_t* lut = reinterpret_cast<uint16_t*>(pqo + kBN);  // 2 c(i - j), below 2^16: span <= 16384
 
   const int nqt = (a.M + kBM - 1) / kBM;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
   }
 
   const int dmin = q0 - (kt_end * kBN - 1);
-  deb_fill_lut(a, lut, a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vt));
+  deb_fill_lut(a, reinterpret_cast<int16_t*>(lut), a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vt));
 
   const uint16_t* Qp = reinterpret_cast<const uint16_t*>(a.q) + b * a.qs[0] + h * a.qs[1];
   const uint16_t* Kp = reinterpret_cast<const uint16_t*>(a.k) + b * a.ks[0] + h * a.ks[1];
@@ -324,7 +324,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
       add_terms(s0, 0, col);
       add_terms(s1, 1, col);
     } else {
-      const int16_t* lp = lut + (lut_lane - key0);
+      const uint16_t* lp = lut + (lut_lane - key0);
       auto col = [&](int e) { return (int)lp[-x_key(e, 0)]; };
       add_terms(s0, 0, col);
       add_terms(s1, 1, col);
@@ -1048,7 +1048,7 @@ extern "C" int vfk_flash_deberta_fwd(const vfk_tensor* q, const vfk_tensor* k, c
   };
   const size_t slds = deb_staged_lds(a.lut_len);
   if (a.unit && (a.pk || a.pq) && (!a.pk || rows16(a.pk, a.pks)) && (!a.pq || rows16(a.pq, a.pqs)) &&
-      a.span % 4 == 0 && 2 * a.span >= kPqW && slds <= 64 * 1024) {
+      a.span % 4 == 0 && 2 * a.span >= kPqW && a.span <= 16384 && slds <= 64 * 1024) {
 #define VFK_DEB_STAGED(E)                                                                         \
   if (a.pk && a.pq)                                                                               \
     hipLaunchKernelGGL((deberta_gather_staged_kernel<E, true, true>), grid, dim3(256), slds, st, a); \
