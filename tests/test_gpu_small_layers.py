@@ -76,6 +76,11 @@ def test_small_layers_refuse(dev):
     with torch.autocast("cuda", torch.float16):
         assert not mb._small_layers(x, cu, w, 2)
     assert not mb._small_layers(x.float(), cu, w, 2)
+    # the token limit, and the work limit of wider layers
+    wide = _weights(1024, 2624, torch.bfloat16, 5).to(dev)
+    for wt, T, want in ((w, 4096, True), (w, 4097, False), (wide, 1600, True), (wide, 1700, False)):
+        rows = torch.zeros(T, wt.hidden, dtype=torch.bfloat16, device=dev)
+        assert mb._small_layers(rows, cu, wt, 2) is want, (wt.hidden, T)
 
 
 def test_small_layers_captured(dev):

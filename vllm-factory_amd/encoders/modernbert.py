@@ -127,6 +127,11 @@ def _dense_ln_fusable(wo: torch.Tensor) -> bool:
 # 2.8 (seven calls are bound by the host there), 5549 3.2 against 3.0, 13090
 # 5.7 against 5.0 (the large tiles of the library products win).
 _SMALL_TOKENS = 4096
+# Wider layers reach that point earlier: what the seven calls cost the host is
+# the same, what the small tiles take grows with a token's products. 28 layers
+# of width 1024, intermediate 2624, ms, one call a layer against seven: 1600
+# tokens 3.0 against 3.5, 2400 3.9 against 3.6 (the line lies at 1676).
+_SMALL_WORK = _SMALL_TOKENS * (4 * 768 * 768 + 3 * 768 * 1152)
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
@@ -135,7 +140,8 @@ def _small_layers(x: torch.Tensor, cu_seqlens: torch.Tensor, w: ModernBertWeight
     weights of x's type on its device with aligned rows, heads of 64, no
     autocast (which would choose another type for the products)."""
     D, dt, dev = w.hidden, x.dtype, x.device
-    if (not 0 < x.shape[0] <= _SMALL_TOKENS or dt not in (torch.bfloat16, torch.float16)
+    if (not 0 < x.shape[0] <= _SMALL_TOKENS
+            or x.shape[0] * D * (4 * D + 3 * w.inter) > _SMALL_WORK or dt not in (torch.bfloat16, torch.float16)
             or torch.is_autocast_enabled() or D != 64 * w.heads or w.inter % 64 or w.inter < 64
             or not x.is_contiguous() or x.data_ptr() % 16
             or cu_seqlens.dtype != torch.int32 or cu_seqlens.dim() != 1 or cu_seqlens.device != dev
