@@ -120,12 +120,12 @@ def test_unaligned_rows(dev):
     assert (out.cpu().double() - want).abs().max() <= ATOL
 
 
-@pytest.mark.parametrize("span", [8192, 9000, 16384])
+@pytest.mark.parametrize("span", [8192, 9000, 16384, 16385, 20000, 32767, 32768])
 def test_deberta_16bit_wide_span(dev, span):
-    """Linear buckets of a wide span: twice a column index takes all 16 bits
-    of the 16-bit kernels' tables. Columns in reach carry the terms, the rest
-    hold 1000, which a wrapped index would pick up. Bound: the oracle's values
-    at this path's tolerance."""
+    """Linear buckets of a wide span: twice a column index (up to 16384) or the
+    index itself (above) takes all 16 bits of the 16-bit kernels' tables.
+    Columns in reach carry the terms, the rest hold 1000, which a wrapped index
+    would pick up. Bound: the oracle's values at this path's tolerance."""
     from _tol import assert_attn_close
     from kernels.flash_deberta_attention import flash_deberta_attention
     g = torch.Generator().manual_seed(span)

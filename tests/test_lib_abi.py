@@ -440,3 +440,25 @@ def test_varlen_direct_rule_and_errors():
     for bad in (dict(scale=0.0), dict(q=q.float(), out=q.float())):
         with pytest.raises(NotImplementedError):
             f(**bad)
+
+
+def test_deberta_dropin_span_limits():
+    """16-bit position terms over more than 2^16 columns are refused before any
+    launch (the kernel's column table is unsigned 16 bits), and spans whose
+    column count does not fit 32 bits in every type."""
+    from kernels import _lib
+    d = lambda t: _lib.ref(_lib.desc(t))
+
+    def f(dt, span, cols, key=True, query=True):
+        q = torch.zeros(1, 1, 8, 64, dtype=dt)
+        pos = torch.zeros(1, 1, 8, 1, dtype=dt).expand(1, 1, 8, cols)
+        _lib.call("vfk_flash_deberta_fwd", d(q), d(q), d(q), None, d(pos if key else None),
+                  d(pos if query else None), 0, 0.125, 0, span, 0, d(q), None)
+    for dt in (torch.bfloat16, torch.float16):
+        for which in (dict(), dict(key=False), dict(query=False)):
+            with pytest.raises(NotImplementedError, match="above 32768"):
+                f(dt, 32769, 65538, **which)
+    with pytest.raises(NotImplementedError, match="too large"):
+        f(torch.float32, 1 << 30, 1 << 32)
+    with pytest.raises(ValueError, match="expected"):
+        f(torch.float32, 1 << 30, 8)

@@ -63,24 +63,28 @@ __device__ inline int deb_index_lds(const DebArgs& a, const int16_t* thr, int d)
   return min(max((d < 0 ? -mag : mag) + a.span, 0), 2 * a.span - 1);
 }
 
-// lut[e] := mul c(dmin + e) (its low 16 bits) for e < n by a 256-thread workgroup. The binary
+// lut[e] := mul c(dmin + e), below 2^16, for e < n by a 256-thread workgroup. The binary
 // search runs over a copy of the thresholds in thr (LDS, VFK_MAX_THR int16,
 // free for other use after the caller's next barrier): its eight or nine
 // dependent reads are LDS reads of about 0.05 us, where reads of the kernel's
 // arguments are cache reads of several times that, two or three times over
 // per workgroup before its first tile.
-__device__ inline void deb_fill_lut(const DebArgs& a, int16_t* lut, int n, int dmin, int mul, int16_t* thr) {
+__device__ inline void deb_fill_lut(const DebArgs& a, uint16_t* lut, int n, int dmin, int mul, int16_t* thr) {
   for (int e = threadIdx.x; e < a.step.nthr; e += 256) thr[e] = a.step.thr[e];
   __syncthreads();
-  for (int e = threadIdx.x; e < n; e += 256) lut[e] = (int16_t)(mul * deb_index_lds(a, thr, dmin + e));
+  for (int e = threadIdx.x; e < n; e += 256) lut[e] = (uint16_t)(mul * deb_index_lds(a, thr, dmin + e));
 }
+
+// Largest span of deberta_gather_kernel with position terms: its columns, up
+// to 2 span - 1, lie in a table of unsigned 16 bits.
+constexpr int kGatherMaxSpan = 32768;
 
 template <typename E>
 __global__ __launch_bounds__(256, 2) void deberta_gather_kernel(DebArgs a) {
   extern __shared__ __align__(16) unsigned char smem[];
   uint16_t* Ks = reinterpret_cast<uint16_t*>(smem);
   uint16_t* Vt = Ks + kKsElems;
-  int16_t* lut = reinterpret_cast<int16_t*>(Vt + kVtElems);  // c(i - j)
+  uint16_t* lut = Vt + kVtElems;  // c(i - j), below 2^16: span <= kGatherMaxSpan
 
   const int nqt = (a.M + kBM - 1) / kBM;
   const int work = xcd_remap(blockIdx.x, gridDim.x);
@@ -138,7 +142,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_kernel(DebArgs a) {
 
     f32x16_t s0, s1;
     qk_tile<E>(Ks, qf, s0, s1);
-    const int16_t* lp = lut + (lut_lane - key0);
+    const uint16_t* lp = lut + (lut_lane - key0);
     map_scores(s0, s1, [&](int e, float v) {
       const int xk = x_key(e, 0);           // key - key0 - 4*hl
       const int key = key0 + xk + 4 * hl;
@@ -226,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
   }
 
   const int dmin = q0 - (kt_end * kBN - 1);
-  deb_fill_lut(a, reinterpret_cast<int16_t*>(lut), a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vt));
+  deb_fill_lut(a, lut, a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vt));
 
   const uint16_t* Qp = reinterpret_cast<const uint16_t*>(a.q) + b * a.qs[0] + h * a.qs[1];
   const uint16_t* Kp = reinterpret_cast<const uint16_t*>(a.k) + b * a.ks[0] + h * a.ks[1];
@@ -600,7 +604,7 @@ __global__ __launch_bounds__(256, 2) void deberta_fused_kernel(DebArgs a) {
   }
   const int kt_end = (len + kBN - 1) / kBN;
   const int dmin = q0 - (kt_end * kBN - 1);
-  deb_fill_lut(a, lut, a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vs));
+  deb_fill_lut(a, reinterpret_cast<uint16_t*>(lut), a.lut_len, dmin, 2, reinterpret_cast<int16_t*>(Vs));
 
   const uint16_t* Qp = reinterpret_cast<const uint16_t*>(a.q) + qb + h * a.qs[1];
   TileSrc ksrc, vsrc;
@@ -987,8 +991,11 @@ static int check_pos(const vfk_tensor* p, const char* name, const DebArgs& a, in
   int rc = check_tensor(p, name, 4);
   if (rc) return rc;
   if (p->dtype != dt) return set_error(VFK_ERR_INVALID, "%s: dtype differs from q", name);
-  if (p->size[0] != a.B || p->size[1] != a.H || p->size[2] != rows || p->size[3] < 2 * a.span)
-    return set_error(VFK_ERR_INVALID, "%s: expected [B, H, %d, >= %d]", name, rows, 2 * a.span);
+  const int64_t cols = 2 * (int64_t)a.span;
+  if (p->size[0] != a.B || p->size[1] != a.H || p->size[2] != rows || p->size[3] < cols)
+    return set_error(VFK_ERR_INVALID, "%s: expected [B, H, %d, >= %lld]", name, rows, (long long)cols);
+  if (cols >= (1ll << 31))  // columns are 32-bit indices
+    return set_error(VFK_ERR_UNSUPPORTED, "%s: att_span %d too large", name, a.span);
   return VFK_OK;
 }
 
@@ -1034,6 +1041,8 @@ extern "C" int vfk_flash_deberta_fwd(const vfk_tensor* q, const vfk_tensor* k, c
   if (a.B == 0 || a.H == 0 || a.M == 0) return VFK_OK;
   hipStream_t st = (hipStream_t)stream;
   if (q->dtype == VFK_F32) return deb_gather_f32_launch(a, st, "vfk_flash_deberta_fwd");
+  if ((a.pk || a.pq) && a.span > kGatherMaxSpan)
+    return set_error(VFK_ERR_UNSUPPORTED, "vfk_flash_deberta_fwd: att_span above %d in 16-bit types", kGatherMaxSpan);
   const int ntk = ceil_div(a.N, kBN);
   a.lut_len = ntk * kBN + kBM;
   const size_t lds = (size_t)(kKsElems + kVtElems) * 2 + (size_t)a.lut_len * 2;
