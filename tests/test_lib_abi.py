@@ -4,6 +4,7 @@ the oracle. No GPU compute is issued here."""
 import ctypes
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -462,3 +463,33 @@ def test_deberta_dropin_span_limits():
         f(torch.float32, 1 << 30, 1 << 32)
     with pytest.raises(ValueError, match="expected"):
         f(torch.float32, 1 << 30, 8)
+
+
+def test_small_product_slices_stay_in_their_row(tmp_path):
+    """Every K slice that the wave groups of a small product load lies inside
+    the row, for every count of slices, and every slice below K is the one
+    that its group multiplies (compiled from the kernels' own function)."""
+    src, exe = tmp_path / "slices.cpp", tmp_path / "slices"
+    src.write_text("""
+#include <stdio.h>
+#include "vfk_host.h"
+int main() {
+  for (int groups = 1; groups <= 4; groups *= 4)
+    for (int nk = 1; nk <= 1024; ++nk)
+      for (int s = 0; s < (nk + groups - 1) / groups; ++s)
+        for (int g = 0; g < groups; ++g) {
+          const int k = vfk::k_slice(s, g, groups, nk);
+          if (k < 0 || k >= nk) return printf("groups %d nk %d: slice %d\\n", groups, nk, k), 1;
+          if (s * groups + g < nk && k != s * groups + g) return printf("groups %d nk %d: moved\\n", groups, nk), 1;
+        }
+  return 0;
+}
+""")
+    csrc = os.path.join(ROOT, "vllm-factory_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-I", csrc, str(src), "-o", str(exe)], check=True)
+    r = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
+    assert r.returncode == 0, r.stdout
+    # and the kernel takes its slices from it alone
+    text = open(os.path.join(csrc, "gemm_small.h")).read()
+    loads = re.findall(r"lds_load16\([xw]r,.*?\);", text, re.S)
+    assert len(loads) == 2 and all("k_slice(" in t for t in loads)

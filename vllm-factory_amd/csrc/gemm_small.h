@@ -185,9 +185,10 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
   const int nk = a.K >> 6, steps = (nk + WK - 1) / WK;
 
   // rows past the end of x or w read as zeros (GLU features past I of the
-  // input half read gate rows, whose products are not stored); the resources
-  // end with the last row's K values, so that the slices past K of a last
-  // step, which no wave multiplies, stay inside them too
+  // input half read gate rows, whose products are not stored); slices stay
+  // inside K (k_slice): the range check takes the scalar offset off a
+  // resource's size, which for a tile of one or two rows is below the offset
+  // of a slice past K
   const int64_t xrows = a.M - t0 < TM ? a.M - t0 : TM;
   const rsrc_t xr = uniform_rsrc(a.x + t0 * (a.xs2 >> 1), (int)(xrows - 1) * a.xs2 + 2 * a.K);
   const rsrc_t wr = uniform_rsrc(a.w, ((GLU ? 2 : 1) * a.I - 1) * a.ws2 + 2 * a.K);
@@ -205,10 +206,10 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
   auto load = [&](int s, char* st) {
 #pragma unroll
     for (int j = 0; j < NX; ++j)
-      lds_load16(xr, st + (4 * j + w) * 1024, vx[j], (s * WK + 32 * j / TM) * 128);
+      lds_load16(xr, st + (4 * j + w) * 1024, vx[j], k_slice(s, 32 * j / TM, WK, nk) * 128);
 #pragma unroll
     for (int j = 0; j < NW; ++j)
-      lds_load16(wr, st + kX + (4 * j + w) * 1024, vw[j], (s * WK + 32 * j / TW) * 128);
+      lds_load16(wr, st + kX + (4 * j + w) * 1024, vw[j], k_slice(s, 32 * j / TW, WK, nk) * 128);
   };
 #pragma unroll
   for (int s = 0; s < ST - 1; ++s)

@@ -39,6 +39,14 @@ VFK_HD inline int step_eval(const StepFn& s, int a) {
   return s.f0 + lo;
 }
 
+// The 64-wide K slice (of nk) that wave group `group` of `groups` loads in a
+// step of a product whose groups share the K slices. The last step can reach
+// past K; such a group loads the last slice again and multiplies nothing, so
+// that no load leaves its row.
+VFK_HD constexpr int k_slice(int step, int group, int groups, int nk) {
+  return step * groups + group < nk ? step * groups + group : nk - 1;
+}
+
 int set_error(int code, const char* fmt, ...);
 
 // T5 bucket of rel = key - query (fp32 reference formula).
