@@ -406,14 +406,19 @@ def test_modernbert_layer_argument_errors():
     wq, wo, wi, wm = z(192, 64), z(64, 64), z(128, 64), z(64, 64)
     fake = 1 << 20
 
-    def f(x=x, pending=None, an=None, wqkv=wq, mn=n, wi=wi, xo=out, rope=fake, ws=fake, size=1 << 30):
+    def f(x=x, pending=None, an=None, wqkv=wq, mn=n, wi=wi, xo=out, rope=fake, ws=fake, size=1 << 30, cu=fake,
+          seqs=1, max_len=4, window=-1, npos=1 << 24, scale=0.125):
         _lib.call("vfk_modernbert_layer_fwd", d(x), d(pending), d(an), d(wqkv), d(wo), d(mn), d(wi), d(wm),
-                  1e-5, fake, 1, 4, -1, rope, 256, None, 0.125, ws, size, d(xo), d(pend), None)
+                  1e-5, cu, seqs, max_len, window, rope, npos, None, scale, ws, size, d(xo), d(pend), None)
     for bad in (dict(xo=x), dict(wqkv=z(192, 128)), dict(mn=z(65)), dict(mn=n.float()), dict(wi=z(128, 65)),
-                dict(rope=None), dict(ws=None), dict(size=16), dict(xo=z(4, 128)), dict(an=z(32))):
+                dict(rope=None), dict(ws=None), dict(size=16), dict(xo=z(4, 128)), dict(an=z(32)), dict(xo=pend),
+                # the attention's, which comes second in the layer
+                dict(cu=None), dict(seqs=0), dict(seqs=-1), dict(max_len=0), dict(npos=3), dict(rope=fake + 4)):
         with pytest.raises(ValueError):
             f(**bad)
-    for bad in (dict(x=z(4, 64, dt=torch.float32)), dict(x=z(4, 65)), dict(wi=z(120, 64)), dict(pending=pend)):
+    for bad in (dict(x=z(4, 64, dt=torch.float32)), dict(x=z(4, 65)), dict(wi=z(120, 64)), dict(pending=pend),
+                dict(scale=0.0), dict(max_len=300, window=65), dict(max_len=(1 << 24) + 1, npos=1 << 25),
+                dict(max_len=1 << 24, seqs=1 << 20, size=1 << 62)):
         with pytest.raises(NotImplementedError):
             f(**bad)
 

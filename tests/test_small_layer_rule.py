@@ -1,0 +1,42 @@
+"""Which ModernBERT calls take one entry point a layer (_small_layers): what the
+entry point refuses and the separate kernels accept must stay with them. The
+rule looks at shapes, types and scalars alone, so it runs without a GPU."""
+import torch
+
+from encoders import modernbert as mb
+
+
+def _weights(D=128, I=64, layers=2, meta=False):
+    dev = "meta" if meta else "cpu"
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
+    ls = [mb.ModernBertLayerWeights(z(3 * D, D), z(D, D), z(2 * I, D), z(D, I), None if i == 0 else z(D), z(D))
+          for i in range(layers)]
+    return mb.ModernBertWeights(D, D // 64, I, z(8, D), z(D), ls, z(D))
+
+
+def _rows(w, T=8):
+    return torch.zeros(T, w.hidden, dtype=torch.bfloat16, device=w.emb.device)
+
+
+def _cu(w, *ends):
+    return torch.tensor(ends, dtype=torch.int32).to(w.emb.device)
+
+
+def test_empty_calls_keep_the_separate_kernels(monkeypatch):
+    """No sequences or a max_seqlen of 0: the entry point refuses them."""
+    w = _weights()
+    assert mb._small_layers(_rows(w), _cu(w, 0, 8), w, 2)
+    assert not mb._small_layers(_rows(w), _cu(w, 0), w, 2)
+    taken = []
+    monkeypatch.setattr(mb, "fused_layernorm", lambda x, *a: x)
+    monkeypatch.setattr(mb, "_small_layers", lambda *a: True)
+    monkeypatch.setattr(mb, "_encode_small", lambda *a: taken.append(a) or (None, a[0]))
+    monkeypatch.setattr(mb.F, "linear", lambda *a: (_ for _ in ()).throw(LookupError))
+    ids = torch.zeros(8, dtype=torch.int64)
+    mb._encode(ids, _cu(w, 0, 8), 8, w, 2)
+    assert len(taken) == 1
+    try:
+        mb._encode(ids, _cu(w, 0, 8), 0, w, 2)
+    except LookupError:
+        pass
+    assert len(taken) == 1

@@ -803,6 +803,44 @@ static int varlen_setup(VarlenArgs& a, const vfk_tensor* q, const vfk_tensor* k,
   return VFK_OK;
 }
 
+// Head pairs per block of the key pre-pass: 4 where H is a multiple of 8 but
+// not of 12, else 6.
+static int pack_pairs(int H) { return (H % 8 == 0 && H % 12 != 0) ? 4 : 6; }
+
+// Blocks of the key pre-pass.
+static int64_t pack_blocks(const VarlenArgs& a) {
+  const int64_t ngrp = (int64_t)ceil_div(a.maxlen, 64) * (64 / kPackRows);
+  return a.nseq * ngrp * ceil_div(a.H, 2 * pack_pairs(a.H));
+}
+
+// Limits of the 16-bit kernels, all before the first launch. Leaves a.window
+// at -1 where the window covers every pair.
+static int varlen_limits(VarlenArgs& a, const char* nm) {
+  // buffer resources cover max_seqlen rows of one slice: byte sizes < 2^31
+  const int64_t span = (int64_t)a.maxlen * 2;
+  if (span * std::max<int64_t>(a.ks[0], 64) >= (1ll << 31) || span * a.vs[0] >= (1ll << 31))
+    return set_error(VFK_ERR_UNSUPPORTED, "%s: max_seqlen x row stride too large", nm);
+  if (a.window >= a.maxlen) a.window = -1;
+  if (a.window > kPenOff - kBM)
+    return set_error(VFK_ERR_UNSUPPORTED, "%s: window %d > %d", nm, a.window, kPenOff - kBM);
+  if ((int64_t)ceil_div(a.maxlen, kBM) * a.H * a.nseq >= (1ll << 31) ||
+      (a.rope && pack_blocks(a) >= (1ll << 31)))
+    return set_error(VFK_ERR_UNSUPPORTED, "%s: grid too large", nm);
+  return VFK_OK;
+}
+
+int vfk::varlen_attn_check(const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,
+                           const int32_t* cu_seqlens, int32_t num_seqs, int32_t max_seqlen, int32_t window,
+                           const float* rope_cos_sin, int32_t rope_positions, float softmax_scale,
+                           vfk_tensor* out, const char* nm) {
+  VarlenArgs a = {};
+  const int rc = varlen_setup(a, q, k, v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin,
+                              rope_positions, nullptr, softmax_scale, out);
+  if (rc) return rc;
+  if (a.nseq == 0) return set_error(VFK_ERR_INVALID, "%s: no sequences", nm);
+  return varlen_limits(a, nm);
+}
+
 extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
                                    const vfk_tensor* v, const int32_t* cu_seqlens,
                                    int32_t num_seqs, int32_t max_seqlen,
@@ -823,10 +861,7 @@ extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
     hipLaunchKernelGGL(varlen_fwd_f32_kernel, dim3((unsigned)blocks), dim3(64), 0, st, a);
     return launch_status("vfk_varlen_attn_fwd");
   }
-  // buffer resources cover max_seqlen rows of one slice: byte sizes < 2^31
-  const int64_t span = (int64_t)max_seqlen * 2;
-  if (span * std::max<int64_t>(a.ks[0], 64) >= (1ll << 31) || span * a.vs[0] >= (1ll << 31))
-    return set_error(VFK_ERR_UNSUPPORTED, "vfk_varlen_attn_fwd: max_seqlen x row stride too large");
+  if ((rc = varlen_limits(a, "vfk_varlen_attn_fwd"))) return rc;
   const bool rope = a.rope != nullptr;
   if (rope) {
     const int64_t need = vfk_varlen_attn_workspace_bytes(dt, T, (int32_t)H, 1, num_seqs, max_seqlen);
@@ -840,12 +875,9 @@ extern "C" int vfk_varlen_attn_fwd(const vfk_tensor* q, const vfk_tensor* k,
     a.nkt = nkt;
     a.kmax = reinterpret_cast<float*>(static_cast<char*>(workspace) + kr_bytes(T, H));
     const int ngrp = nkt * (64 / kPackRows);
-    // 4 head pairs per block where H is a multiple of 8 but not of 12, else 6
-    const int npair = (H % 8 == 0 && H % 12 != 0) ? 4 : 6;
-    const int nhg = (int)ceil_div(H, 2 * npair);
-    const int64_t pblocks = (int64_t)num_seqs * ngrp * nhg;
-    if (pblocks >= (1ll << 31))
-      return set_error(VFK_ERR_UNSUPPORTED, "vfk_varlen_attn_fwd: grid too large");
+    const int npair = pack_pairs((int)H);
+    const int nhg = ceil_div(H, 2 * npair);
+    const int64_t pblocks = pack_blocks(a);
 #define VFK_PACK(E, NP) \
   hipLaunchKernelGGL((rope_k_pack_kernel<E, NP>), dim3((unsigned)pblocks), dim3(256), 0, st, a, ngrp, nhg)
     if (dt == VFK_BF16) {
@@ -879,13 +911,8 @@ extern "C" int vfk_varlen_attn_direct_fwd(const vfk_tensor* q, const vfk_tensor*
   if (q->dtype == VFK_F32) return set_error(VFK_ERR_UNSUPPORTED, "%s: bf16 or fp16 only", nm);
   if (!rope_cos_sin) return set_error(VFK_ERR_INVALID, "%s: rope table missing", nm);
   if (a.nseq == 0) return VFK_OK;
-  if (a.window >= max_seqlen) a.window = -1;  // window covers every pair
   // as the other form, so that a call does not depend on the one it takes
-  if (a.window > kPenOff - kBM)
-    return set_error(VFK_ERR_UNSUPPORTED, "%s: window %d > %d", nm, a.window, kPenOff - kBM);
-  const int64_t span = (int64_t)max_seqlen * 2;  // buffer resource of the V rows
-  if (span * a.ks[0] >= (1ll << 31) || span * a.vs[0] >= (1ll << 31))
-    return set_error(VFK_ERR_UNSUPPORTED, "%s: max_seqlen x row stride too large", nm);
+  if ((rc = varlen_limits(a, nm))) return rc;
   a.nqt = ceil_div(max_seqlen, kDirRows);
   const int64_t blocks = (int64_t)a.nqt * a.H * num_seqs;
   if (blocks >= (1ll << 31)) return set_error(VFK_ERR_UNSUPPORTED, "%s: grid too large", nm);

@@ -49,4 +49,12 @@ inline int launch_status(const char* what) {
 
 inline int ceil_div(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 
+// What vfk_varlen_attn_fwd would refuse in these 16-bit arguments (and no
+// sequences or no keys), without a launch: for an entry point that enqueues
+// other kernels in front of the attention.
+int varlen_attn_check(const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,
+                      const int32_t* cu_seqlens, int32_t num_seqs, int32_t max_seqlen, int32_t window,
+                      const float* rope_cos_sin, int32_t rope_positions, float softmax_scale,
+                      vfk_tensor* out, const char* nm);
+
 }  // namespace vfk

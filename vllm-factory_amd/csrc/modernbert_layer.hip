@@ -148,6 +148,8 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
   if (!rope_cos_sin) return set_error(VFK_ERR_INVALID, "%s: rope table missing", nm);
   // the column of workgroups that writes x_out runs beside others that read x
   if (x_out->data == x->data) return set_error(VFK_ERR_INVALID, "%s: x_out must not be x", nm);
+  if (x_out->data == pending_out->data)
+    return set_error(VFK_ERR_INVALID, "%s: x_out must not be pending_out", nm);
   if (M > (1 << 20)) return set_error(VFK_ERR_UNSUPPORTED, "%s: too many tokens", nm);
   if (M == 0) return VFK_OK;
   const LayerBuffers buf(M, D, I,
@@ -155,6 +157,14 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
   if (!workspace || workspace_bytes < buf.total || !aligned16(workspace))
     return set_error(VFK_ERR_INVALID, "%s: workspace needs %lld 16-byte aligned bytes", nm, (long long)buf.total);
   char* ws = static_cast<char*>(workspace);
+  const int64_t H = D / 64;
+  uint16_t* qkv = reinterpret_cast<uint16_t*>(ws + buf.qkv);
+  const vfk_tensor q = heads3(qkv, dt, M, 3 * D, H), k = heads3(qkv + D, dt, M, 3 * D, H),
+                   v = heads3(qkv + 2 * D, dt, M, 3 * D, H);
+  vfk_tensor att = heads3(ws + buf.att, dt, M, D, H);
+  if ((rc = varlen_attn_check(&q, &k, &v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin,
+                              rope_positions, softmax_scale, &att, nm)))
+    return rc;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int cus = compute_units();
   const bool norm_fits = D <= kNormMaxK;
@@ -181,11 +191,6 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
     else project<F16, kActPlain>(a, fused, small, st);
     if ((rc = launch_status(nm))) return rc;
   }
-  const int64_t H = D / 64;
-  uint16_t* qkv = reinterpret_cast<uint16_t*>(ws + buf.qkv);
-  const vfk_tensor q = heads3(qkv, dt, M, 3 * D, H), k = heads3(qkv + D, dt, M, 3 * D, H),
-                   v = heads3(qkv + 2 * D, dt, M, 3 * D, H);
-  vfk_tensor att = heads3(ws + buf.att, dt, M, D, H);
   // the split keys are summed in another order than one chain sums them: as
   // with the split K of the products, only where those split K too, so that a
   // sequence of more tokens gives the same bits alone and in a large pack

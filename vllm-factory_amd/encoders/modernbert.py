@@ -145,7 +145,7 @@ def _small_layers(x: torch.Tensor, cu_seqlens: torch.Tensor, w: ModernBertWeight
             or torch.is_autocast_enabled() or D != 64 * w.heads or w.inter % 64 or w.inter < 64
             or not x.is_contiguous() or x.data_ptr() % 16
             or cu_seqlens.dtype != torch.int32 or cu_seqlens.dim() != 1 or cu_seqlens.device != dev
-            or not cu_seqlens.is_contiguous() or n == 0):
+            or not cu_seqlens.is_contiguous() or cu_seqlens.numel() < 2 or n == 0):
         return False
     shapes = ((3 * D, D), (D, D), (2 * w.inter, D), (D, w.inter), (D,), (D,))
     for i in range(n):
@@ -210,7 +210,7 @@ def _encode(ids: torch.Tensor, cu_seqlens: torch.Tensor, max_seqlen: int, w: Mod
     x = fused_layernorm(w.emb[ids], w.hidden, w.emb_norm, None, w.eps)
     pending = None  # MLP output not yet added to the residual stream x
     n = len(w.layers) if num_layers is None else num_layers
-    if not (fuse_qkv_rope or fuse_dense_ln) and _small_layers(x, cu_seqlens, w, n):
+    if not (fuse_qkv_rope or fuse_dense_ln) and max_seqlen > 0 and _small_layers(x, cu_seqlens, w, n):
         return _encode_small(x, cu_seqlens, max_seqlen, key_valid, w, n)
     positions = None  # rotary position of each token, for the fused q | k | v projection
     for i in range(n):
