@@ -100,3 +100,15 @@ def test_small_layers_captured(dev):
         got = out.clone()
         assert torch.equal(got, call())
         torch.cuda.synchronize()
+
+
+def test_small_layers_without_rotation(dev):
+    """theta 0: no rotation in that kind of layer (bound as above)."""
+    for field in ("theta_global", "theta_local"):
+        w = _weights(128, 192, torch.bfloat16, 6)
+        setattr(w, field, 0.0)
+        ids = torch.randint(0, 100, (90,), generator=torch.Generator().manual_seed(2))
+        cu = torch.tensor([0, 40, 90], dtype=torch.int32)
+        want = _want(ids, cu, w)
+        got = mb.modernbert_forward(ids.to(dev), cu.to(dev), 50, w.to(dev)).cpu().double()
+        assert float((got - want).norm() / want.norm()) <= 8.4e-3

@@ -40,3 +40,12 @@ def test_empty_calls_keep_the_separate_kernels(monkeypatch):
     except LookupError:
         pass
     assert len(taken) == 1
+
+
+def test_no_rotary_embedding_keeps_the_separate_kernels():
+    """theta <= 0 means no rotation, which the entry point does not have."""
+    for field in ("theta_global", "theta_local"):
+        for theta in (0.0, -1.0):
+            w = _weights()
+            setattr(w, field, theta)
+            assert not mb._small_layers(_rows(w), _cu(w, 0, 8), w, 2)

@@ -137,11 +137,13 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 def _small_layers(x: torch.Tensor, cu_seqlens: torch.Tensor, w: ModernBertWeights, n: int) -> bool:
     """Whether the layers take vfk_modernbert_layer_fwd: few tokens, 16-bit
-    weights of x's type on its device with aligned rows, heads of 64, no
-    autocast (which would choose another type for the products)."""
+    weights of x's type on its device with aligned rows, heads of 64, rotary
+    embedding in every layer, no autocast (which would choose another type for
+    the products)."""
     D, dt, dev = w.hidden, x.dtype, x.device
     if (not 0 < x.shape[0] <= _SMALL_TOKENS
             or x.shape[0] * D * (4 * D + 3 * w.inter) > _SMALL_WORK or dt not in (torch.bfloat16, torch.float16)
+            or not (w.theta_global > 0 and w.theta_local > 0)  # 0: no rotation
             or torch.is_autocast_enabled() or D != 64 * w.heads or w.inter % 64 or w.inter < 64
             or not x.is_contiguous() or x.data_ptr() % 16
             or cu_seqlens.dtype != torch.int32 or cu_seqlens.dim() != 1 or cu_seqlens.device != dev
