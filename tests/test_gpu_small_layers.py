@@ -112,3 +112,16 @@ def test_small_layers_without_rotation(dev):
         want = _want(ids, cu, w)
         got = mb.modernbert_forward(ids.to(dev), cu.to(dev), 50, w.to(dev)).cpu().double()
         assert float((got - want).norm() / want.norm()) <= 8.4e-3
+
+
+@pytest.mark.parametrize("n", [0, -1])
+def test_no_layers(dev, n):
+    """No layer runs: the normed embeddings, whatever memory held before."""
+    w = _weights(128, 64, torch.bfloat16, 7).to(dev)
+    ids = torch.randint(0, 100, (50,), generator=torch.Generator().manual_seed(3)).to(dev)
+    cu = torch.tensor([0, 50], dtype=torch.int32, device=dev)
+    junk = torch.full((50, 128), float("nan"), dtype=torch.bfloat16, device=dev)
+    del junk  # what an uninitialised buffer would show
+    got = mb.modernbert_forward(ids, cu, 50, w, num_layers=n)
+    x = mb.fused_layernorm(w.emb[ids], 128, w.emb_norm, None, w.eps)
+    assert torch.equal(got, mb.fused_layernorm(x, 128, w.final_norm, None, w.eps))

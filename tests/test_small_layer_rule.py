@@ -49,3 +49,11 @@ def test_no_rotary_embedding_keeps_the_separate_kernels():
             w = _weights()
             setattr(w, field, theta)
             assert not mb._small_layers(_rows(w), _cu(w, 0, 8), w, 2)
+
+
+def test_no_layers_keep_the_separate_kernels():
+    """Without a layer (num_layers 0, or below, which runs none either) there
+    is no MLP output to add."""
+    w = _weights()
+    for n in (0, -1, -2):
+        assert not mb._small_layers(_rows(w), _cu(w, 0, 8), w, n)

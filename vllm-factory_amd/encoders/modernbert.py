@@ -147,7 +147,7 @@ def _small_layers(x: torch.Tensor, cu_seqlens: torch.Tensor, w: ModernBertWeight
             or torch.is_autocast_enabled() or D != 64 * w.heads or w.inter % 64 or w.inter < 64
             or not x.is_contiguous() or x.data_ptr() % 16
             or cu_seqlens.dtype != torch.int32 or cu_seqlens.dim() != 1 or cu_seqlens.device != dev
-            or not cu_seqlens.is_contiguous() or cu_seqlens.numel() < 2 or n == 0):
+            or not cu_seqlens.is_contiguous() or cu_seqlens.numel() < 2 or n <= 0):
         return False
     shapes = ((3 * D, D), (D, D), (2 * w.inter, D), (D, w.inter), (D,), (D,))
     for i in range(n):
