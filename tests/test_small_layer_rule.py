@@ -57,3 +57,21 @@ def test_no_layers_keep_the_separate_kernels():
     w = _weights()
     for n in (0, -1, -2):
         assert not mb._small_layers(_rows(w), _cu(w, 0, 8), w, n)
+
+
+def test_sizes_beyond_the_entry_point_keep_the_separate_kernels():
+    """Widths the entry point refuses, few tokens: hidden above 16384,
+    intermediate above 65536, a weight of 2 GiB. (Meta tensors: sizes only.)"""
+    for D, I, T, want in ((16384, 64, 4, True), (16448, 64, 4, False), (64, 65536, 8, True), (64, 65600, 8, False),
+                          (8192, 65472, 2, False), (16384, 32768, 2, False), (16384, 32640, 2, True)):
+        w = _weights(D, I, meta=True)
+        assert mb._small_layers(_rows(w, T), _cu(w, 0, T), w, 2) is want, (D, I)
+
+
+def test_the_entry_point_takes_what_the_rule_lets_through():
+    """Every weight of a size that the rule accepts lies within the entry
+    point's offsets: (rows + 128) rows of it below 2 GiB."""
+    for D in range(64, 16385, 64):
+        I = min(65536, (mb._MAX_WEIGHT - 1) // (4 * D) // 64 * 64)
+        for rows, cols in ((3 * D, D), (D, D), (2 * I, D), (D, I)):
+            assert 2 * (rows + 128) * cols < 1 << 31, (D, I)

@@ -133,6 +133,10 @@ _SMALL_TOKENS = 4096
 # tokens 3.0 against 3.5, 2400 3.9 against 3.6 (the line lies at 1676).
 _SMALL_WORK = _SMALL_TOKENS * (4 * 768 * 768 + 3 * 768 * 1152)
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+# Bytes of wi (4 I D) from which the entry point's 32-bit offsets, which reach
+# one tile of rows past a weight, do not hold it; with hidden <= 16384 they hold
+# the other weights.
+_MAX_WEIGHT = (1 << 31) - 256 * 16384
 
 
 def _small_layers(x: torch.Tensor, cu_seqlens: torch.Tensor, w: ModernBertWeights, n: int) -> bool:
@@ -145,6 +149,7 @@ def _small_layers(x: torch.Tensor, cu_seqlens: torch.Tensor, w: ModernBertWeight
             or x.shape[0] * D * (4 * D + 3 * w.inter) > _SMALL_WORK or dt not in (torch.bfloat16, torch.float16)
             or not (w.theta_global > 0 and w.theta_local > 0)  # 0: no rotation
             or torch.is_autocast_enabled() or D != 64 * w.heads or w.inter % 64 or w.inter < 64
+            or D > 16384 or w.inter > 65536 or 4 * D * w.inter >= _MAX_WEIGHT
             or not x.is_contiguous() or x.data_ptr() % 16
             or cu_seqlens.dtype != torch.int32 or cu_seqlens.dim() != 1 or cu_seqlens.device != dev
             or not cu_seqlens.is_contiguous() or cu_seqlens.numel() < 2 or n <= 0):
