@@ -498,3 +498,37 @@ int main() {
     text = open(os.path.join(csrc, "gemm_small.h")).read()
     loads = re.findall(r"lds_load16\([xw]r,.*?\);", text, re.S)
     assert len(loads) == 2 and all("k_slice(" in t for t in loads)
+
+
+def test_descriptions_are_checked_arguments():
+    """An entry point's tensor argument takes a description: an address or
+    another object in its place is an error of the call, not memory that is
+    read, and so is a description in a scalar's place. desc() packs the fields
+    of vfk_tensor."""
+    from kernels import _lib
+
+    class Tensor(ctypes.Structure):  # include/vfk.h
+        _fields_ = [("data", ctypes.c_void_p), ("dtype", ctypes.c_int32), ("ndim", ctypes.c_int32),
+                    ("size", ctypes.c_int64 * 4), ("stride", ctypes.c_int64 * 4)]
+
+    def fields(*a, **k):
+        b = _lib.desc(*a, **k)
+        assert len(b) == ctypes.sizeof(Tensor)
+        d = Tensor.from_buffer_copy(b)
+        return d.data, d.dtype, d.ndim, list(d.size), list(d.stride)
+    t = torch.zeros(3, 5, 7, dtype=torch.float16)[:, 1:]
+    assert fields(t) == (t.data_ptr(), _lib.F16, 3, [3, 4, 7, 1], [35, 7, 1, 0])
+    assert fields(t, shape=[12, 7], strides=[7, 1]) == (t.data_ptr(), _lib.F16, 2, [12, 7, 1, 1], [7, 1, 0, 0])
+    assert _lib.ref(_lib.desc(None)) is None
+    with pytest.raises(ValueError, match="at most 4 dims"):
+        _lib.desc(torch.zeros(1, 1, 1, 1, 1))
+    x = _lib.ref(_lib.desc(torch.zeros(4, 8)))
+    for wrong in (t.data_ptr(), ctypes.c_void_p(t.data_ptr()), ctypes.byref(ctypes.c_int64(0)), "x", t):
+        with pytest.raises(ctypes.ArgumentError):
+            _lib.call("vfk_act_fwd", 77, wrong, x, None)
+        with pytest.raises(ctypes.ArgumentError):
+            _lib.call("vfk_act_fwd", 77, x, wrong, None)
+    with pytest.raises(ctypes.ArgumentError):
+        _lib.call("vfk_act_fwd", x, x, x, None)
+    with pytest.raises(ValueError):  # an unknown activation: the descriptions themselves pass
+        _lib.call("vfk_act_fwd", 77, x, x, None)

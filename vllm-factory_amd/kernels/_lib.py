@@ -1,7 +1,7 @@
 """ctypes binding of libvfk.so (the gfx950 kernel library, C ABI in include/vfk.h).
 
 Every public op in this package goes through `call()`: tensors are described by
-packed `VfkTensor` structures (pointer, dtype code, sizes, element strides) and
+packed vfk_tensor structures (pointer, dtype code, sizes, element strides) and
 kernels run on the caller's current torch stream. There is no CPU or alternative GPU path: a
 missing library or a non-GPU tensor raises.
 """
@@ -25,19 +25,12 @@ ACT_GELU_ERF, ACT_GELU_TANH, ACT_SILU, ACT_RELU = 0, 1, 2, 3
 _DTYPE_CODE = {torch.float32: F32, torch.bfloat16: BF16, torch.float16: F16}
 
 
-class VfkTensor(ctypes.Structure):
-    _fields_ = [
-        ("data", ctypes.c_void_p),
-        ("dtype", ctypes.c_int32),
-        ("ndim", ctypes.c_int32),
-        ("size", ctypes.c_int64 * 4),
-        ("stride", ctypes.c_int64 * 4),
-    ]
-
-
-_PACK = struct.Struct("@Pii8q").pack  # a VfkTensor as bytes
+_PACK = struct.Struct("@Pii8q").pack  # vfk_tensor: data, dtype, ndim, size[4], stride[4]
 _vp = ctypes.c_void_p
-_P = _vp  # a VfkTensor: the bytes that desc() packs, or a reference to a structure
+# A vfk_tensor: the bytes that desc() packs. Of the types that take bytes this
+# one refuses integers, so that an address in a tensor's place is an error of
+# the call and not memory that is read as a description.
+_P = ctypes.c_char_p
 _i32 = ctypes.c_int32
 _f32 = ctypes.c_float
 _i64 = ctypes.c_int64
@@ -145,7 +138,7 @@ _ONES, _ZEROS = (1, 1, 1, 1), (0, 0, 0, 0)
 def desc(t: Optional[torch.Tensor], shape: Optional[Sequence[int]] = None,
          strides: Optional[Sequence[int]] = None) -> Optional[bytes]:
     """Describes a tensor (optionally with an overriding view shape/strides):
-    the bytes of a VfkTensor, valid for the length of the call they go to."""
+    the bytes of a vfk_tensor, valid for the length of the call they go to."""
     if t is None:
         return None
     if shape is None:
