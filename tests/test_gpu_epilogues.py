@@ -426,3 +426,16 @@ def test_packed_weights_under_inference_mode(dev):
                                        round_dtype=torch.bfloat16)
         err = (y.float().cpu() - ref).abs().max().item()
         assert err <= 6e-2 and cosine(y.float().cpu(), ref) >= 0.9999, err
+
+
+@pytest.mark.parametrize("rms", [False, True])
+@pytest.mark.parametrize("shape", [(3, 2, 64), (6, 64), (12, 32), (3, 128), (1, 384), (384,)])
+def test_residual_of_another_shape(dev, rms, shape):
+    """A residual of as many values as x counts as rows of x's width whatever
+    its shape: the same bits as the residual laid out like x."""
+    from kernels.fused_layernorm import fused_add_layernorm
+    from kernels.rms_norm import fused_add_rms_norm
+    x, r, w = (_rand(s, torch.bfloat16, 90 + i).to(dev) for i, s in enumerate([(6, 64), (6, 64), (64,)]))
+    call = (lambda r: fused_add_rms_norm(x, r, w)) if rms else (lambda r: fused_add_layernorm(x, r, w, None, 1e-5))
+    for got, want in zip(call(r.reshape(shape)), call(r)):
+        assert got.shape == x.shape and torch.equal(got, want)
