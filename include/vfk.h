@@ -512,8 +512,9 @@ int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_tensor* w,
 
 /* vfk_varlen_attn_fwd with RoPE for few queries: the keys are rotated where
  * they are used, without a pre-pass and its workspace, and the waves of a
- * workgroup split them. Same arguments and results to rounding; bf16 / fp16,
- * rope table required. vfk_varlen_attn_direct: 1 where this form is the
+ * workgroup split them. Same arguments and results to rounding, but out must
+ * not overlap k, which vfk_varlen_attn_fwd copies first; bf16 / fp16, rope
+ * table required. vfk_varlen_attn_direct: 1 where this form is the
  * faster one. */
 int vfk_varlen_attn_direct(int32_t dtype, int32_t num_heads, int32_t num_seqs, int32_t max_seqlen);
 int vfk_varlen_attn_direct_fwd(const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,

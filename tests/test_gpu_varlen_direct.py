@@ -55,3 +55,20 @@ def test_direct_cuts_at_max_seqlen(dev):
     cu2 = torch.tensor([0, 40, 80], dtype=torch.int32, device=dev)
     want = va.varlen_rope_attention(cut[:, 0], cut[:, 1], cut[:, 2], cu2, 40, -1, 10000.0, 0.125)
     assert torch.equal(torch.cat([got[:40], got[50:]]), want)
+
+
+@pytest.mark.parametrize("which", [0, 1])
+def test_output_in_place(dev, which, monkeypatch):
+    """out may be q or k: a short call then gives what it gives through the
+    pre-pass, which copies k before anything is written."""
+    g = torch.Generator().manual_seed(11)
+    qkv = torch.randn(300, 3, 12, 64, generator=g).bfloat16().to(dev)
+    cu = torch.tensor([0, 300], dtype=torch.int32, device=dev)
+    call = lambda t, out: va.varlen_rope_attention(t[:, 0], t[:, 1], t[:, 2], cu, 300, -1, 10000.0, 0.125, out=out)
+    lib = _lib.load()
+    assert lib.vfk_varlen_attn_direct(_lib.BF16, 12, 1, 300) == 1
+    with monkeypatch.context() as m:
+        m.setattr(lib, "vfk_varlen_attn_direct", lambda *a: 0)
+        want = call(qkv, None)
+    t = qkv.clone()
+    assert torch.equal(call(t, t[:, which]), want)

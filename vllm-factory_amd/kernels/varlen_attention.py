@@ -66,6 +66,9 @@ def varlen_rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if not cu_seqlens.is_contiguous():
         cu_seqlens = cu_seqlens.contiguous()
     qq, kk, vv = (_lib.rows_aligned(t) for t in (q, k, v))
+    # out may be k: the pre-pass has rotated k into its workspace by then; the
+    # form without it reads k until its last workgroup is done
+    fresh = out is None or out.untyped_storage().data_ptr() != kk.untyped_storage().data_ptr()
     if out is None:
         out = q.new_empty(q.shape)
     kv_ptr = None
@@ -80,8 +83,8 @@ def varlen_rope_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     if rope:
         tab = rope_table(rope_theta, int(max_seqlen), dev)
         tab_ptr, tab_n = tab.data_ptr(), tab.shape[0]
-        if _lib.load().vfk_varlen_attn_direct(_lib.dtype_code(q.dtype), q.shape[1], cu_seqlens.numel() - 1,
-                                              int(max_seqlen)):
+        if fresh and _lib.load().vfk_varlen_attn_direct(_lib.dtype_code(q.dtype), q.shape[1],
+                                                        cu_seqlens.numel() - 1, int(max_seqlen)):
             # few queries: keys rotated in the attention kernel, no workspace
             _lib.on_device(
                 "vfk_varlen_attn_direct_fwd", dev,
