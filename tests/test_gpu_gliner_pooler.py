@@ -342,3 +342,27 @@ def test_span_marker_forward_matches_oracle():
     cs = cosine(got, want)
     print(f"span marker: max-abs {err:.3e} (scale {scale:.3f}) cosine {cs:.6f}", flush=True)
     assert err <= 2e-2 * scale and cs >= 0.9999, (err, scale, cs)
+
+
+@pytest.mark.parametrize("D", [64, 20, 33])
+@pytest.mark.parametrize("columns", [False, True])
+def test_span_marker_halves_of_w1(D, columns, monkeypatch):
+    """The halves of the first weight reach the products on 16-byte boundaries
+    at every width and order of w1's memory, as views with aligned rows or as
+    copies (bf16 sums of at most 64 terms: 2e-2 of the scale)."""
+    import kernels.gliner_pooler as gp
+    g = torch.Generator().manual_seed(D)
+    rnd = lambda *s: torch.randn(*s, generator=g).bfloat16().cuda()
+    start, end, w1 = rnd(9, D), rnd(9, D), rnd(64, 2 * D)
+    w1 = w1.t().contiguous().t() if columns else w1
+    seen, got = [], []
+    matmul = torch.matmul
+    monkeypatch.setattr(torch, "matmul", lambda x, y: seen.append(y) or matmul(x, y))
+    monkeypatch.setattr(gp, "gliner_span_hidden", lambda a, b, *r: got.extend([a, b]) or a)
+    gp.span_marker_forward(start, end, None, None, None, None, w1, None, rnd(8, 64), None)
+    for y, x, h in zip(seen, (start, end), (0, D)):
+        w = y.t()
+        assert w.data_ptr() % 16 == 0 and (w.is_contiguous() or w.stride(0) * 2 % 16 == 0)
+        assert torch.equal(w, w1[:, h:h + D])
+        want = x.float().relu() @ w1[:, h:h + D].float().t()
+        assert (got[h > 0].float() - want).abs().max() <= 2e-2 * want.abs().max()

@@ -271,9 +271,10 @@ def span_marker_forward(start_rep: torch.Tensor, end_rep: torch.Tensor, row_cu: 
     if w1.shape[1] != 2 * D:
         raise ValueError("w1 must be [4D, 2D] for start/end rows of width D")
     from .activation import activation
-    # the halves of w1 go to the products as they lie (row stride 2D)
-    a = torch.matmul(activation(start_rep, "relu"), w1[:, :D].t())
-    b = torch.matmul(activation(end_rep, "relu"), w1[:, D:].t())
+    # the halves of w1 go to the products as they lie (row stride 2D) where
+    # their rows are 16-byte aligned, else as copies
+    a = torch.matmul(activation(start_rep, "relu"), _lib.rows_aligned(w1[:, :D]).t())
+    b = torch.matmul(activation(end_rep, "relu"), _lib.rows_aligned(w1[:, D:]).t())
     h = gliner_span_hidden(a, b, b1, row_cu, span_idx, span_mask, span_cu)
     if b2 is None:
         return torch.matmul(h, w2.t())
