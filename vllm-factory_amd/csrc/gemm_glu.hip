@@ -444,7 +444,7 @@ __global__ __launch_bounds__(256, 1) void gemm_glu_kernel(GluArgs a) {
 }
 
 // The tiles of gemm_small.h for the arguments of a GLU launch.
-template <typename E, int WM, int WN, int WK, int ST>
+template <typename E, int WM, int WN, int WK>
 void launch_glu_small(int act, const GluArgs& g, hipStream_t st) {
   SmallArgs a = {};
   a.x = g.x; a.w = g.w; a.out = g.out;
@@ -452,16 +452,16 @@ void launch_glu_small(int act, const GluArgs& g, hipStream_t st) {
   a.xs2 = g.xs2; a.ws2 = g.ws2; a.os = g.os;
   switch (act) {
     case VFK_ACT_GELU_ERF:
-      launch_gemm_small<E, VFK_ACT_GELU_ERF, false, 2, WM, WN, WK, ST>(a, st);
+      launch_gemm_small<E, VFK_ACT_GELU_ERF, false, 2, WM, WN, WK>(a, st);
       break;
     case VFK_ACT_GELU_TANH:
-      launch_gemm_small<E, VFK_ACT_GELU_TANH, false, 2, WM, WN, WK, ST>(a, st);
+      launch_gemm_small<E, VFK_ACT_GELU_TANH, false, 2, WM, WN, WK>(a, st);
       break;
     case VFK_ACT_SILU:
-      launch_gemm_small<E, VFK_ACT_SILU, false, 2, WM, WN, WK, ST>(a, st);
+      launch_gemm_small<E, VFK_ACT_SILU, false, 2, WM, WN, WK>(a, st);
       break;
     default:
-      launch_gemm_small<E, VFK_ACT_RELU, false, 2, WM, WN, WK, ST>(a, st);
+      launch_gemm_small<E, VFK_ACT_RELU, false, 2, WM, WN, WK>(a, st);
       break;
   }
 }
@@ -576,13 +576,13 @@ extern "C" int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_te
   const int cus = compute_units();
   const GluTile tile = glu_tile(a, cus);
   if (tile == GLU_32) {
-    if (dt == VFK_BF16) launch_glu_small<BF16, 1, 1, 4, 3>(act, a, st);
-    else launch_glu_small<F16, 1, 1, 4, 3>(act, a, st);
+    if (dt == VFK_BF16) launch_glu_small<BF16, 1, 1, 4>(act, a, st);
+    else launch_glu_small<F16, 1, 1, 4>(act, a, st);
     return launch_status("glu_linear");
   }
   if (tile == GLU_64) {
-    if (dt == VFK_BF16) launch_glu_small<BF16, 2, 2, 1, 3>(act, a, st);
-    else launch_glu_small<F16, 2, 2, 1, 3>(act, a, st);
+    if (dt == VFK_BF16) launch_glu_small<BF16, 2, 2, 1>(act, a, st);
+    else launch_glu_small<F16, 2, 2, 1>(act, a, st);
     return launch_status("glu_linear");
   }
   const int grid = persistent_grid(a, cus);

@@ -7,7 +7,7 @@
 // 500 at I = 1152, each of which walks all of K alone while the rest of the
 // chip idles. Here a workgroup owns 32 WM tokens x 32 WN NB weight rows (GLU:
 // NB = 2, the input and the gate rows of 32 WN features), four waves as WM x
-// WN x WK: the same calls give 36 and 144 workgroups, and ST stages keep ST - 1
+// WN x WK: the same calls give 36 and 144 workgroups, and three stages keep two
 // steps of loads in flight, so that the time is about a memory latency plus
 // the slices. GLU: 19.9 -> 5.5 us and 24.3 -> 7.3 us (six stages of 64 x 64,
 // one workgroup a CU instead of two: 8.3 us).
@@ -33,6 +33,7 @@ namespace vfk {
 
 constexpr int kActPlain = -1;   // no GLU: out = x W^T
 constexpr int kNormMaxK = 1024;
+constexpr int kStages = 3;      // LDS stages of a product
 
 struct SmallArgs {
   const uint16_t* x;
@@ -158,7 +159,7 @@ __device__ inline void norm_rows32(const SmallArgs& a, int64_t t0, bool write_su
   }
 }
 
-template <typename E, int ACT, bool NORM, int NB, int WM, int WN, int WK, int ST>
+template <typename E, int ACT, bool NORM, int NB, int WM, int WN, int WK>
 __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
   constexpr bool GLU = ACT != kActPlain;
   constexpr int TM = 32 * WM, TF = 32 * WN, TW = NB * TF;  // tokens, features, weight rows
@@ -166,10 +167,10 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
   constexpr int NX = NORM ? 0 : WK * TM / 32, NW = WK * TW / 32;  // 8-row loads of a wave per stage
   constexpr int L = NX + NW;
   constexpr int kNorm = NORM ? kNormMaxK * 64 : 0;  // normalised rows, after the stages
-  static_assert(WM * WN * WK == 4 && (ST - 2) * L <= 63 && ST >= 2 && ST <= 6, "shape");
+  static_assert(WM * WN * WK == 4 && (kStages - 2) * L <= 63, "shape");
   static_assert((!GLU || NB == 2) && (!NORM || WK == 4), "form");
-  static_assert(ST * kStage >= NB * 16384, "the partial sums of the K groups");
-  __shared__ __attribute__((aligned(1024))) char smem[ST * kStage + kNorm];
+  static_assert(kStages * kStage >= NB * 16384, "the partial sums of the K groups");
+  __shared__ __attribute__((aligned(1024))) char smem[kStages * kStage + kNorm];
   const int l = threadIdx.x & 63, c = l & 31, h = l >> 5;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wk = WK == 4 ? w : 0, wm = WK == 4 ? 0 : w / WN, wn = WK == 4 ? 0 : w % WN;
@@ -212,10 +213,10 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
       lds_load16(wr, st + kX + (4 * j + w) * 1024, vw[j], k_slice(s, 32 * j / TW, WK, nk) * 128);
   };
 #pragma unroll
-  for (int s = 0; s < ST - 1; ++s)
+  for (int s = 0; s < kStages - 1; ++s)
     if (s < steps) load(s, smem + s * kStage);
   if (NORM) {
-    norm_rows32<E>(a, t0, ni == 0 && a.sum, smem + ST * kStage);
+    norm_rows32<E>(a, t0, ni == 0 && a.sum, smem + kStages * kStage);
     // the loop's waits count loads, which return in order; stores need not
     if (ni == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
@@ -228,18 +229,13 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
     xo[ds] = o + (wk * TM + 32 * wm) * 128;
     wo[ds] = o + kX + (wk * TW + 32 * wn) * 128;
   }
-  int cur = 0, nxt = (ST - 1) * kStage;  // stage offsets of step s and of step s + ST - 1
+  int cur = 0, nxt = (kStages - 1) * kStage;  // stage offsets of step s and of step s + kStages - 1
   for (int s = 0; s < steps; ++s) {
-    // step s has landed in every wave, and every wave is done with step s - 1
-    switch (min(ST - 2, steps - 1 - s)) {
-      case 0: step_barrier<0>(); break;
-      case 1: step_barrier<(ST > 2 ? 1 : 0) * L>(); break;
-      case 2: step_barrier<(ST > 3 ? 2 : 0) * L>(); break;
-      case 3: step_barrier<(ST > 4 ? 3 : 0) * L>(); break;
-      default: step_barrier<(ST > 5 ? 4 : 0) * L>(); break;
-    }
+    // step s has landed in every wave, and every wave is done with step s - 1;
+    // the loads of step s + 1, if there is one, stay in flight
+    if (s + 1 < steps) step_barrier<L>(); else step_barrier<0>();
     const char* st = smem + cur;
-    const char* xs = NORM ? smem + ST * kStage + s * WK * 4096 : st;
+    const char* xs = NORM ? smem + kStages * kStage + s * WK * 4096 : st;
     u32x4_t xf[4], wf[NB][4];
 #pragma unroll
     for (int ds = 0; ds < 4; ++ds) {
@@ -249,9 +245,9 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
         wf[g][ds] = *reinterpret_cast<const u32x4_t*>(st + wo[ds] + g * TF * 128);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (s + ST - 1 < steps) load(s + ST - 1, smem + nxt);
-    cur = cur == (ST - 1) * kStage ? 0 : cur + kStage;
-    nxt = nxt == (ST - 1) * kStage ? 0 : nxt + kStage;
+    if (s + kStages - 1 < steps) load(s + kStages - 1, smem + nxt);
+    cur = cur == (kStages - 1) * kStage ? 0 : cur + kStage;
+    nxt = nxt == (kStages - 1) * kStage ? 0 : nxt + kStage;
     if (WK == 1 || s * WK + wk < nk) {  // uniform in the wave
 #pragma unroll
       for (int ds = 0; ds < 4; ++ds)
@@ -308,12 +304,12 @@ __global__ __launch_bounds__(256) void gemm_small_kernel(SmallArgs a) {
   put(w, y);
 }
 
-template <typename E, int ACT, bool NORM, int NB, int WM, int WN, int WK, int ST>
+template <typename E, int ACT, bool NORM, int NB, int WM, int WN, int WK>
 inline void launch_gemm_small(SmallArgs& a, hipStream_t st) {
   const int tf = 32 * WN * (ACT != kActPlain ? 1 : NB);
   a.mt = (int)((a.M + 32 * WM - 1) / (32 * WM));
   a.nt = (a.I + tf - 1) / tf;
-  gemm_small_kernel<E, ACT, NORM, NB, WM, WN, WK, ST><<<a.mt * a.nt, 256, 0, st>>>(a);
+  gemm_small_kernel<E, ACT, NORM, NB, WM, WN, WK><<<a.mt * a.nt, 256, 0, st>>>(a);
 }
 
 inline int compute_units() {

@@ -53,14 +53,17 @@ vfk_tensor heads3(void* p, int dt, int64_t M, int64_t row, int64_t H) {
   return t;
 }
 
-// out = x w^T, optionally after LayerNorm(x + res) (norm != nullptr: the 32 x
-// 32 tiles only).
+// out = x w^T on the 32 x 32 tiles or the 64 x 128 ones.
+template <typename E>
+void project(SmallArgs a, bool small, hipStream_t st) {
+  if (small) launch_gemm_small<E, kActPlain, false, 1, 1, 1, 4>(a, st);
+  else launch_gemm_small<E, kActPlain, false, 2, 2, 2, 1>(a, st);
+}
+
+// out = LayerNorm(x + res) w^T, or its GLU, on the 32 x 32 tiles.
 template <typename E, int ACT>
-void project(SmallArgs a, bool norm, bool small, hipStream_t st) {
-  constexpr int NB32 = ACT == kActPlain ? 1 : 2;
-  if (norm) launch_gemm_small<E, ACT, true, NB32, 1, 1, 4, 3>(a, st);
-  else if (small) launch_gemm_small<E, ACT, false, NB32, 1, 1, 4, 3>(a, st);
-  else launch_gemm_small<E, ACT, false, 2, 2, 2, 1, 3>(a, st);
+void project_norm(SmallArgs a, hipStream_t st) {
+  launch_gemm_small<E, ACT, true, ACT == kActPlain ? 1 : 2, 1, 1, 4>(a, st);
 }
 
 SmallArgs small_args(const void* x, int64_t xs, const vfk_tensor* w, void* out, int64_t os, int64_t M,
@@ -187,8 +190,10 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
       a.x = static_cast<const uint16_t*>(h.data);
     }
     if (!has_pending) x1.data = x->data;
-    if (dt == VFK_BF16) project<BF16, kActPlain>(a, fused, small, st);
-    else project<F16, kActPlain>(a, fused, small, st);
+    if (fused && dt == VFK_BF16) project_norm<BF16, kActPlain>(a, st);
+    else if (fused) project_norm<F16, kActPlain>(a, st);
+    else if (dt == VFK_BF16) project<BF16>(a, small, st);
+    else project<F16>(a, small, st);
     if ((rc = launch_status(nm))) return rc;
   }
   // the split keys are summed in another order than one chain sums them: as
@@ -206,8 +211,8 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
   const bool narrow = tiles32_fit(M, D, cus);
   {
     const SmallArgs a = small_args(att.data, D, wo, o.data, D, M, D);
-    if (dt == VFK_BF16) project<BF16, kActPlain>(a, false, narrow, st);
-    else project<F16, kActPlain>(a, false, narrow, st);
+    if (dt == VFK_BF16) project<BF16>(a, narrow, st);
+    else project<F16>(a, narrow, st);
     if ((rc = launch_status(nm))) return rc;
   }
   // g = GELU(input) * gate of LayerNorm(x1 + o); x_out = x1 + o
@@ -217,8 +222,8 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
     a.rs = D; a.ss = D; a.eps = eps;
     a.sum = static_cast<uint16_t*>(x_out->data);
     a.nw = static_cast<const uint16_t*>(mlp_norm->data);
-    if (dt == VFK_BF16) project<BF16, VFK_ACT_GELU_ERF>(a, true, true, st);
-    else project<F16, VFK_ACT_GELU_ERF>(a, true, true, st);
+    if (dt == VFK_BF16) project_norm<BF16, VFK_ACT_GELU_ERF>(a, st);
+    else project_norm<F16, VFK_ACT_GELU_ERF>(a, st);
     if ((rc = launch_status(nm))) return rc;
   } else {
     if ((rc = vfk_layernorm_fwd(&o, &x1, mlp_norm, nullptr, eps, &h, x_out, stream)) ||
@@ -226,7 +231,7 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
       return rc;
   }
   const SmallArgs a = small_args(g.data, I, wo_mlp, pending_out->data, D, M, D);
-  if (dt == VFK_BF16) project<BF16, kActPlain>(a, false, narrow, st);
-  else project<F16, kActPlain>(a, false, narrow, st);
+  if (dt == VFK_BF16) project<BF16>(a, narrow, st);
+  else project<F16>(a, narrow, st);
   return launch_status(nm);
 }
