@@ -506,7 +506,13 @@ int vfk_glu_fwd(int32_t act, const vfk_tensor* a, const vfk_tensor* b,
  * (ModernBertMLP.forward up to Wo) and the T5 gated FF's wi_0 / wi_1 products
  * (models/mt5/mt5_encoder.py T5DenseGatedActDense); kernels/fused_glu_mlp.py:61-104
  * is the elementwise part. bf16 / fp16; rows contiguous and 16-byte aligned;
- * K a multiple of 64, I a multiple of 8. */
+ * K a multiple of 64, I a multiple of 8.
+ * vfk_glu_linear_tile: tokens of the tile that a call of `rows` rows and I =
+ * `features` takes on the current device (0: no rows). Tiles of 64 and 256
+ * tokens sum K in one order, so that a row has the same bits alone and among
+ * others; tiles of 32 (few rows: up to 224 at I = 1152 and 256 compute units)
+ * add four partial sums and agree with them to rounding. */
+int vfk_glu_linear_tile(int64_t rows, int32_t features);
 int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_tensor* w,
                        vfk_tensor* out, void* stream);
 
@@ -514,8 +520,10 @@ int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_tensor* w,
  * they are used, without a pre-pass and its workspace, and the waves of a
  * workgroup split them. Same arguments and results to rounding, but out must
  * not overlap k, which vfk_varlen_attn_fwd copies first; bf16 / fp16, rope
- * table required. vfk_varlen_attn_direct: 1 where this form is the
- * faster one. */
+ * table required. vfk_varlen_attn_direct: 1 where a call is the faster this
+ * way (12 heads: one sequence of up to 512 tokens, 16 of up to 128). A sequence
+ * of such a call agrees with itself in a larger pack to rounding, not bit for
+ * bit as between packs that both take the pre-pass. */
 int vfk_varlen_attn_direct(int32_t dtype, int32_t num_heads, int32_t num_seqs, int32_t max_seqlen);
 int vfk_varlen_attn_direct_fwd(const vfk_tensor* q, const vfk_tensor* k, const vfk_tensor* v,
                                const int32_t* cu_seqlens, int32_t num_seqs, int32_t max_seqlen,
@@ -535,7 +543,13 @@ int vfk_varlen_attn_direct_fwd(const vfk_tensor* q, const vfk_tensor* k, const v
  * and I multiples of 64, D / 64 heads. x_out must not be x. The attention's
  * arguments are those of vfk_varlen_attn_fwd. The workspace takes
  * vfk_modernbert_layer_workspace_bytes and may be shared by the layers of one
- * stream. */
+ * stream.
+ * Where a product's 32 x 32 tiles have a compute unit each, its K is split
+ * over four waves, and up to the line of Wqkv the attention is the direct
+ * form where that is the faster one. At width 768, intermediate 1152 and 256
+ * compute units that is up to 96 tokens for Wqkv, 224 for Wi and 320 for Wo
+ * and the MLP output: a sequence of up to 320 tokens alone agrees with itself
+ * in a larger pack to rounding, a longer call bit for bit. */
 int64_t vfk_modernbert_layer_workspace_bytes(int32_t dtype, int64_t tokens, int32_t hidden,
                                              int32_t inter, int32_t num_seqs, int32_t max_seqlen);
 int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* pending,

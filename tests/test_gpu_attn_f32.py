@@ -118,26 +118,3 @@ def test_unaligned_rows(dev):
     flash_attention_rpb_final(qd, kd, vd, None, 32, 128, False, softmax_scale=0.125, out=out)
     want = oa.rpb_attention(q, k, v, None, 32, 128, False, None, 0.125, dtype=torch.float64)
     assert (out.cpu().double() - want).abs().max() <= ATOL
-
-
-@pytest.mark.parametrize("span", [8192, 9000, 16384, 16385, 20000, 32767, 32768])
-def test_deberta_16bit_wide_span(dev, span):
-    """Linear buckets of a wide span: twice a column index (up to 16384) or the
-    index itself (above) takes all 16 bits of the 16-bit kernels' tables.
-    Columns in reach carry the terms, the rest hold 1000, which a wrapped index
-    would pick up. Bound: the oracle's values at this path's tolerance."""
-    from _tol import assert_attn_close
-    from kernels.flash_deberta_attention import flash_deberta_attention
-    g = torch.Generator().manual_seed(span)
-    L = 70
-    q, k, v = (_rand(g, 1, 1, L, 64).bfloat16() for _ in range(3))
-    pk, pq = (torch.full((1, 1, L, 2 * span), 1000.0) for _ in range(2))
-    for p in (pk, pq):
-        p[..., span - L:span + L] = _rand(g, 1, 1, L, 2 * L)
-    pk, pq = pk.bfloat16(), pq.bfloat16()
-    got = flash_deberta_attention(q.to(dev), k.to(dev), v.to(dev), None, pk.to(dev), pq.to(dev), False, 0.07, 0,
-                                  span, False)
-    # the oracle over the columns in reach (it lays out every one it is given)
-    near = slice(span - 2 * L, span + 2 * L)
-    want = oa.deberta_flash_attention(q, k, v, None, pk[..., near], pq[..., near], 0.07, 0, 2 * L, False)
-    assert_attn_close(got, want, f"span {span}")

@@ -144,7 +144,8 @@ def test_modernbert_config5_full_pack_properties():
     """The whole config-5 pack (256 sequences, T = 163 736) through all 22
     layers: every output is finite, and two sequences run alone give their
     rows of the packed forward bit for bit (no attention across sequence
-    boundaries; the GEMMs compute each row the same way at any row count)."""
+    boundaries; from 321 tokens on every product and attention sums a row in
+    the same order at any row count)."""
     import encoders.modernbert as em
     import workloads
     c = workloads.config5()

@@ -100,17 +100,21 @@ def test_glu_linear_modernbert_config5_shape(dev):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("M,K,I", [
-    (1, 64, 8), (31, 192, 40), (33, 320, 1152), (224, 768, 1152),       # 32 x 32 tiles, K split unevenly
-    (225, 64, 1152), (257, 128, 1160), (500, 768, 1152), (65, 1024, 8200),  # 64 x 64
-    (4600, 128, 1152), (4700, 128, 1152)])                              # the line to 256 x 128
-def test_glu_linear_tiles(dev, dtype, M, K, I):
+@pytest.mark.parametrize("tile,M,K,I", [
+    # K split unevenly over the four waves
+    (32, 1, 64, 8), (32, 31, 192, 40), (32, 33, 320, 1152), (32, 224, 768, 1152),
+    (64, 225, 64, 1152), (64, 257, 128, 1160), (64, 500, 768, 1152), (64, 65, 1024, 8200),
+    # the line to 256 x 128
+    (64, 4600, 128, 1152), (256, 4700, 128, 1152)])
+def test_glu_linear_tiles(dev, dtype, tile, M, K, I):
     """Each tile at its edges: K slices that do not divide among the waves,
     fewer slices than stages, ragged tokens and features; x and w with row
     strides above K, whose gaps and tails must not enter (they hold NaN). The
     bound is the one above."""
+    from kernels import _lib
     from kernels.fused_glu_mlp import glu_linear
     print("glu tiles", dtype, M, K, I, flush=True)
+    assert _lib.load().vfk_glu_linear_tile(M, I) == tile
     x, w = _inputs(M, K, I, dtype, M + K + I)
     xd = torch.full((M, K + 8), float("nan"), dtype=dtype, device=dev)
     wd = torch.full((2 * I, K + 8), float("nan"), dtype=dtype, device=dev)
@@ -121,3 +125,24 @@ def test_glu_linear_tiles(dev, dtype, M, K, I):
     y = xd[:, :K].double() @ wd[:, :K].double().t()
     want = torch.nn.functional.gelu(y[:, :I]) * y[:, I:]
     assert_elem_close(out[:M, :I], want, dtype, f"glu_linear {M}x{K}x{I}")
+
+
+def test_glu_linear_row_alone_and_among_others(dev):
+    """A row has the same bits in the 64- and the 256-token tiles, and agrees
+    to rounding in the 32-token ones, whose four partial sums are added in
+    another order: the fp32 sums differ by 2^-24 times the sum of the terms'
+    sizes (11 here) times the square root of their number (28) at most, times a
+    gate below 5, 1e-4, and one bf16 step."""
+    from kernels import _lib
+    from kernels.fused_glu_mlp import glu_linear
+    x, w = _inputs(6000, 768, 1152, torch.bfloat16, 3)
+    x, w = x.to(dev), w.to(dev)
+    tile = _lib.load().vfk_glu_linear_tile
+    assert [tile(n, 1152) for n in (6000, 500, 225, 224, 32)] == [256, 64, 64, 32, 32]
+    full = glu_linear(x, w, "gelu")
+    for n in (225, 500):
+        assert torch.equal(glu_linear(x[:n], w, "gelu"), full[:n]), n
+    for n in (1, 32, 224):
+        got, want = glu_linear(x[:n], w, "gelu").float(), full[:n].float()
+        step = torch.maximum(got.abs(), want.abs()) * 2 ** -7  # a bf16 step is at most 2^-7 of the value
+        assert ((got - want).abs() <= step + 1e-4).all(), n

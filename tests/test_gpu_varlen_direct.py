@@ -29,6 +29,8 @@ def test_direct_matches_prepass(dev, dtype, lens, window, masked, monkeypatch):
     qkv = torch.randn(T, 3, H, 64, generator=g).to(dtype)
     cu = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32)
     valid = torch.rand(T, generator=g) > 0.3 if masked else None
+    if masked and len(lens) > 1:
+        valid[lens[0]:lens[0] + lens[1]] = False  # rows that see no key are zeros
     d = qkv.to(dev)
     call = lambda: va.varlen_rope_attention(d[:, 0], d[:, 1], d[:, 2], cu.to(dev), max(lens), window, 10000.0,
                                             0.125, None if valid is None else valid.to(dev)).cpu()

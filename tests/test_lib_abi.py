@@ -532,3 +532,15 @@ def test_descriptions_are_checked_arguments():
         _lib.call("vfk_act_fwd", x, x, x, None)
     with pytest.raises(ValueError):  # an unknown activation: the descriptions themselves pass
         _lib.call("vfk_act_fwd", 77, x, x, None)
+
+
+def test_glu_tile_rule():
+    """The rule is a function of rows, features and compute units (256 without
+    a device): 32 tokens while every tile has a unit, 256 past two rounds."""
+    from kernels import _lib
+    tile = _lib.load().vfk_glu_linear_tile
+    if torch.cuda.is_available():
+        pytest.skip("the units of the device decide")
+    assert [tile(n, 1152) for n in (0, 1, 224, 225, 4600, 4700, 160000)] == [0, 32, 32, 64, 64, 256, 256]
+    assert [tile(n, 2816) for n in (64, 65, 3000, 4000)] == [32, 64, 64, 256]
+    assert tile(1 << 40, 65536) == 256 and tile(8, 0) == 0

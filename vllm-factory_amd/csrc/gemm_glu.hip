@@ -505,10 +505,12 @@ int persistent_grid(GluArgs& a, int cus) {
 //    rounds, I = 2816); past the line M = 6000 32.3 against 30.4 and M = 4000
 //    68.8 against 64.9. From three rounds on the large tiles win throughout
 //    (the 64 x 64 tiles read x and w four and two times as often).
-enum GluTile { GLU_32, GLU_64, GLU_256 };
-GluTile glu_tile(const GluArgs& a, int cus) {
-  const auto tiles = [&](int64_t m, int64_t f) { return ((a.M + m - 1) / m) * ((a.I + f - 1) / f); };
-  if (tiles32_fit(a.M, a.I, cus)) return GLU_32;
+// The 64 x 64 and the 256 x 128 tiles sum K in one chain, in the same order: a
+// row has the same bits in either. The 32 x 32 tiles add four partial sums.
+enum GluTile { GLU_32 = 32, GLU_64 = 64, GLU_256 = 256 };  // tokens of a tile
+GluTile glu_tile(int64_t M, int64_t I, int cus) {
+  const auto tiles = [&](int64_t m, int64_t f) { return ((M + m - 1) / m) * ((I + f - 1) / f); };
+  if (tiles32_fit(M, I, cus)) return GLU_32;
   const int64_t rounds = (tiles(kGRows, kGFeat) + cus - 1) / cus;
   if (rounds <= 2 && tiles(64, 64) * 256 <= 1300 * rounds * cus) return GLU_64;
   return GLU_256;
@@ -518,6 +520,11 @@ GluTile glu_tile(const GluArgs& a, int cus) {
 }  // namespace vfk
 
 using namespace vfk;
+
+extern "C" int vfk_glu_linear_tile(int64_t rows, int32_t features) {
+  if (rows <= 0 || features <= 0) return 0;
+  return glu_tile(rows, features, compute_units());
+}
 
 extern "C" int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_tensor* w,
                                   vfk_tensor* out, void* stream) {
@@ -574,7 +581,7 @@ extern "C" int vfk_glu_linear_fwd(int32_t act, const vfk_tensor* x, const vfk_te
   a.nt = (int)nt;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int cus = compute_units();
-  const GluTile tile = glu_tile(a, cus);
+  const GluTile tile = glu_tile(M, I, cus);
   if (tile == GLU_32) {
     if (dt == VFK_BF16) launch_glu_small<BF16, 1, 1, 4>(act, a, st);
     else launch_glu_small<F16, 1, 1, 4>(act, a, st);

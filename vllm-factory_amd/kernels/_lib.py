@@ -73,6 +73,7 @@ _SIGNATURES = {
     "vfk_rmsnorm_fwd": [_P, _P, _P, _f32, _P, _P, _vp],
     "vfk_glu_fwd": [_i32, _P, _P, _P, _vp],
     "vfk_glu_linear_fwd": [_i32, _P, _P, _P, _vp],
+    "vfk_glu_linear_tile": [_i64, _i32],
     "vfk_modernbert_layer_workspace_bytes": [_i32, _i64, _i32, _i32, _i32, _i32],
     "vfk_modernbert_layer_fwd": [_P, _P, _P, _P, _P, _P, _P, _P, _f32, _vp, _i32, _i32, _i32, _vp, _i32,
                                  _vp, _f32, _vp, _i64, _P, _P, _vp],
