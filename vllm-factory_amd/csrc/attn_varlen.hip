@@ -497,10 +497,18 @@ constexpr int kDirPad = 68;  // floats per merged output row
 // Largest product of 128-row items (sequences x heads x query tiles of the
 // longest) and query tiles of a call that takes it, 192: with the number of
 // items the workgroups of 128 rows fill the chip, with the length each row's
-// keys are rotated by more workgroups. Two layers (one global, one local) of
-// 12 heads, us, this form against the other: 1 x 32 tokens 22 against 33, 1 x
-// 300 23 against 33, 8 x 40 23 against 38, 16 x 120 30 against 35; past the
-// line 8 x 250 39 against 36, 2 x 700 50 against 35, 4 x 1100 137 against 55.
+// keys are rotated by more workgroups. us of a global / a local (+-64) layer of
+// 12 heads on the device, pre-pass against this form: 1 x 32 tokens 8.7 / 8.6
+// against 6.8 / 6.8, 1 x 512 14.4 / 12.6 against 11.3 / 8.4, 8 x 128 10.4 / 10.7
+// against 9.6 / 10.2, 16 x 64 9.1 / 9.2 against 8.2 / 8.2, 4 x 256 12.0 / 11.7
+// against 12.5 / 11.7; past the line 2 x 384 13.2 / 12.5 against 16.0 / 10.8, 1 x
+// 700 16.3 / 12.8 against 22.7 / 10.8, 8 x 250 12.1 / 11.8 against 18.6 / 16.4. An
+// eager call is bound by the host, which has one launch and one workspace less
+// to make: 18 us against 12.5 to 15 for either layer wherever the rule takes
+// this form, among them the calls of 400 to 768 workgroups of 32 rows (12 x 100,
+// 16 x 120), whose kernels take 4 us longer (10.6 / 11.1 against 15.3 / 15.1) and
+// which a captured graph would rather have with the pre-pass. The rule does not
+// look at the window: up to its line both layers gain or lose alike.
 constexpr int kDirectMaxWork = 192;
 
 // The wave's 64 V rows from key0 on into its own LDS tile.

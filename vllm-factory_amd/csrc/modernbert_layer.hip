@@ -7,9 +7,10 @@
 // of host time each. Here the products run on the tiles of gemm_small.h; where
 // their 32 x 32 tiles fit the chip, the residual add and the LayerNorm in
 // front of Wqkv and Wi are done by those products themselves, so that a layer
-// is six launches instead of eight. 22 layers of width 768 with the embedding
-// and the head, one query of 32 tokens: 2.81 ms as separate calls, 0.72 as one
-// call a layer (kernels 1.05 -> 0.74 ms, host 2.8 -> 0.57).
+// is six launches instead of eight. 22 layers of width 768 with the embedding,
+// 32 tokens: 2.57 ms as separate calls, 0.71 as one call a layer; on the device
+// alone 0.87 and 0.69 (1.34 with the 256 x 128 GLU tiles). With the ColBERT
+// head, one query: 0.78 ms, its kernels 0.74, the host 0.57.
 #include <math.h>
 
 #include "gemm_small.h"
@@ -196,9 +197,11 @@ extern "C" int vfk_modernbert_layer_fwd(const vfk_tensor* x, const vfk_tensor* p
     else project<F16>(a, small, st);
     if ((rc = launch_status(nm))) return rc;
   }
-  // the split keys are summed in another order than one chain sums them: as
-  // with the split K of the products, only where those split K too, so that a
-  // sequence of more tokens gives the same bits alone and in a large pack
+  // The direct form sums the split keys in another order than one chain does,
+  // as the products that split K do (Wqkv up to this line, Wi and Wo up to
+  // theirs further on). It is taken only with all of them: past this line the
+  // attention gives the bits of a large pack and the products' sums alone make
+  // a difference, past Wo's line (320 tokens at width 768) nothing does.
   if (tiles32_fit(M, 3 * D, cus) && vfk_varlen_attn_direct(dt, (int32_t)H, num_seqs, max_seqlen)) {
     if ((rc = vfk_varlen_attn_direct_fwd(&q, &k, &v, cu_seqlens, num_seqs, max_seqlen, window, rope_cos_sin,
                                          rope_positions, key_valid, softmax_scale, &att, stream)))

@@ -10,7 +10,9 @@ Wqkv and the rotary step of k run as one kernel (qkv_rope_projection), which
 rotates the fp32 projection sums of k and rounds once; the attention then
 reads that rotated k (varlen_rope_attention_krot) with no separate k pass.
 Up to _SMALL_TOKENS tokens a layer is one call (vfk_modernbert_layer_fwd) that
-enqueues the library's own products, norms and attention.
+enqueues the library's own products, norms and attention. Its products of few
+rows split K over four waves: a call of up to 320 tokens (width 768) agrees with
+its rows in a larger pack to rounding, longer calls bit for bit.
 Global layers (layer_id % 3 == 0) attend inside each sequence with RoPE theta
 160000, local layers within |i - j| <= 64 with theta 10000; tokens with id
 50284 are hidden as keys (:456-460).
@@ -121,16 +123,31 @@ def _dense_ln_fusable(wo: torch.Tensor) -> bool:
 
 
 # Token count up to which a layer runs as one call on the library's own small
-# tiles (vfk_modernbert_layer_fwd) instead of seven calls. 22 layers of width
-# 768, ms, one call a layer against seven: 32 tokens 0.72 against 2.9, 300 1.07
-# against 2.8, 1262 1.44 against 2.9, 3147 2.16 against 2.9, 3935 2.5 against
-# 2.8 (seven calls are bound by the host there), 5549 3.2 against 3.0, 13090
-# 5.7 against 5.0 (the large tiles of the library products win).
+# tiles (vfk_modernbert_layer_fwd) instead of seven separate calls. 22 layers of
+# width 768, ms, seven calls / one call a layer, as eager calls and on the
+# device alone (replays of a captured graph, which pay no host time):
+#     32 tokens  2.57 / 0.71  device 0.87 / 0.69
+#    512         2.57 / 1.23         1.08 / 1.21
+#   1024         2.67 / 1.42         1.47 / 1.41
+#   2048         2.68 / 1.84         1.90 / 1.85
+#   2880         2.70 / 2.19         2.10 / 2.16
+#   4096         2.70 / 2.57         2.44 / 2.56
+#   4608         2.70 / 2.80         2.57 / 2.79
+#   5549         2.99 / 3.31         2.98 / 3.29
+#   7853         4.38 / 4.06         4.35 / 4.08
+#  13090         5.22 / 6.12         5.22 / 6.07
+# The line is that of eager calls, which the host bounds up to some 5000 tokens
+# (seven calls issue in 2.6 to 2.9 ms); on the device alone the two are within 6 %
+# of each other from 1000 tokens up to it, and both below the 2.31 and 2.69 ms
+# of 2048 and 4096 tokens with the 256 x 128 GLU tiles alone. The tiles go over
+# the chip in rounds, so the crossing is not monotone: one call is ahead again
+# where the library products begin a round (7853).
 _SMALL_TOKENS = 4096
 # Wider layers reach that point earlier: what the seven calls cost the host is
 # the same, what the small tiles take grows with a token's products. 28 layers
-# of width 1024, intermediate 2624, ms, one call a layer against seven: 1600
-# tokens 3.0 against 3.5, 2400 3.9 against 3.6 (the line lies at 1676).
+# of width 1024, intermediate 2624, ms, seven calls / one call a layer: 1536
+# tokens 3.68 / 3.02 (device 3.01 / 2.98), 2048 3.66 / 3.49 (3.48 / 3.45), 2560
+# 3.79 / 4.01 (3.76 / 3.97); the line lies at 1676.
 _SMALL_WORK = _SMALL_TOKENS * (4 * 768 * 768 + 3 * 768 * 1152)
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 # Bytes of wi (4 I D) from which the entry point's 32-bit offsets, which reach

@@ -45,7 +45,9 @@ def glu_linear(x: torch.Tensor, weight: torch.Tensor, act_fn: str = "gelu",
     the unfused path rounds the projection first.
 
     x [..., K] and weight in bf16 or fp16; K a multiple of 64, I of 8. Returns
-    [..., I] (or fills `out`, a [rows, I] tensor with contiguous rows)."""
+    [..., I] (or fills `out`, a [rows, I] tensor with contiguous rows). Few rows
+    (up to 224 at I = 1152) split K over four waves: such a row agrees with
+    itself among more rows to rounding, from there on bit for bit."""
     dev = _lib.require_gpu(x, weight)
     K = x.shape[-1]
     if weight.dim() != 2 or weight.shape[1] != K or weight.shape[0] % 2:

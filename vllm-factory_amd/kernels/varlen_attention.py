@@ -13,7 +13,9 @@ the same attention per sequence from cu_seqlens:
   * rope_theta > 0: q and k are rotated with the HF ModernBertRotaryEmbedding
     frequencies (non-interleaved halves): k once by a pre-pass into a
     workspace, or, where the call has few queries, inside the attention kernel
-    as q always is (inputs are never written);
+    as q always is (inputs are never written); that kernel splits the keys over
+    its waves, so a sequence of such a call (12 heads: one of up to 512 tokens)
+    agrees with itself in a larger pack to rounding, not bit for bit;
   * key_valid[t] == 0 hides key t (the reference's token-id 50284 mask).
 
 Rows that see no key at all are returned as zeros.
