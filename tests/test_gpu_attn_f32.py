@@ -118,3 +118,25 @@ def test_unaligned_rows(dev):
     flash_attention_rpb_final(qd, kd, vd, None, 32, 128, False, softmax_scale=0.125, out=out)
     want = oa.rpb_attention(q, k, v, None, 32, 128, False, None, 0.125, dtype=torch.float64)
     assert (out.cpu().double() - want).abs().max() <= ATOL
+
+
+@pytest.mark.parametrize("op", ["rpb", "deberta"])
+def test_more_workgroups_than_a_launch_holds(dev, op):
+    """2^24 (batch, head) pairs of one row, the largest count that the entry
+    points take: 2^32 threads, more than one launch holds. One key each, so
+    every row is its batch's V exactly. Inputs are expanded; the output takes
+    4 GiB."""
+    from kernels.flash_attention_rpb import flash_attention_rpb_final
+    from kernels.flash_deberta_attention import flash_deberta_attention
+    print("2^24 heads", op, flush=True)
+    n = 1 << 12
+    q = torch.ones(1, 1, 1, 64, device=dev).expand(n, n, 1, 64)
+    rows = torch.arange(n * 64, dtype=torch.float32, device=dev).view(n, 1, 1, 64)
+    v = rows.expand(n, n, 1, 64)
+    if op == "rpb":
+        got = flash_attention_rpb_final(q, q, v, None, 32, 128, False, softmax_scale=0.125)
+    else:
+        got = flash_deberta_attention(q, q, v, None, None, None, False, 0.125, 16, 64, True)
+    assert got.shape == (n, n, 1, 64)
+    for b0 in range(0, n, 256):
+        assert torch.equal(got[b0:b0 + 256], v[b0:b0 + 256]), b0

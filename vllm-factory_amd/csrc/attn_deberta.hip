@@ -366,6 +366,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_staged_kernel(DebArgs a
 struct DebF32Args {
   int lut;   // LDS table of c
   int sat;   // distance from which c no longer changes
+  int work0; // work item of the launch's first workgroup
 };
 
 template <bool RUN>
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(256, 2) void deberta_gather_f32_kernel(DebArgs a, D
   __shared__ int16_t thr[VFK_MAX_THR];
   extern __shared__ int16_t lutc[];
   const int nqt = (a.M + kF32Rows - 1) / kF32Rows;
-  const int work = xcd_remap(blockIdx.x, gridDim.x);
+  const int work = x.work0 + xcd_remap(blockIdx.x, gridDim.x);
   const int bh = work / nqt, h = bh % a.H, b = bh / a.H;
   const int t = threadIdx.x;
   const int len = a.seq_lengths ? min(max(a.seq_lengths[b], 0), a.N) : a.N;
@@ -1008,11 +1009,15 @@ static int deb_gather_f32_launch(const DebArgs& a, hipStream_t st, const char* n
   const size_t lds = x.lut ? (size_t)std::min(2 * x.sat + 1, a.N + kF32Rows - 1) * 2 : 0;
   const bool run = a.unit && a.pk && a.pks[3] == 1 && a.span >= 2;
 #define VFK_DEB_F32(R, C) \
-  hipLaunchKernelGGL((deberta_gather_f32_kernel<R, C>), dim3((unsigned)grid), dim3(256), lds, st, a, x)
-  if (a.causal) {
-    if (run) VFK_DEB_F32(true, true); else VFK_DEB_F32(false, true);
-  } else {
-    if (run) VFK_DEB_F32(true, false); else VFK_DEB_F32(false, false);
+  hipLaunchKernelGGL((deberta_gather_f32_kernel<R, C>), dim3(n), dim3(256), lds, st, a, x)
+  for (int64_t w0 = 0; w0 < grid; w0 += kF32MaxGrid) {
+    const unsigned n = (unsigned)std::min(kF32MaxGrid, grid - w0);
+    x.work0 = (int)w0;
+    if (a.causal) {
+      if (run) VFK_DEB_F32(true, true); else VFK_DEB_F32(false, true);
+    } else {
+      if (run) VFK_DEB_F32(true, false); else VFK_DEB_F32(false, false);
+    }
   }
 #undef VFK_DEB_F32
   return launch_status(name);

@@ -45,6 +45,10 @@ constexpr int kF32Rows = 16;       // query rows per workgroup
 constexpr int kF32Waves = 4;
 constexpr int kF32Pad = 68;        // floats per merged output row (64 + 4)
 constexpr int kF32MaxLut = 2048;   // largest saturation distance kept as an LDS table
+// Workgroups of one launch, whose threads must stay below 2^32. A call of more
+// (16 rows take the 256 threads that 256 rows take at one thread each) goes in
+// several launches.
+constexpr int64_t kF32MaxGrid = ((1ll << 32) - 1) / (64 * kF32Waves);
 
 struct F32Args {
   const float *q, *k, *v;  // row 0 of this (batch, head)

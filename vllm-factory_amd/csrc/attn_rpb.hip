@@ -32,6 +32,7 @@ struct RpbArgs {
   int bidir, causal, offset_pos;  // offset added for rel > 0 (bidirectional)
   int lut_len;  // ntiles * kBN + kBM (LDS bias table entries); fp32: > 0 when there is a table
   int lut_sat;  // fp32: distance from which the bucket no longer changes
+  int work0;    // fp32: work item of the launch's first workgroup
   StepFn step;
   // packed sequences (nullptr: the padded batch): "batch" b is sequence b,
   // tokens cu[b] .. cu[b + 1] - 1 of [T, H, D] tensors (strides [.][1] =
@@ -399,7 +400,7 @@ __global__ __launch_bounds__(256, 2) void rpb_fwd_f32_kernel(RpbArgs a) {
   __shared__ int16_t thr[VFK_MAX_THR];
   extern __shared__ float lutf[];
   const int nqt = (a.Lq + kF32Rows - 1) / kF32Rows;
-  const int work = xcd_remap(blockIdx.x, gridDim.x);
+  const int work = a.work0 + xcd_remap(blockIdx.x, gridDim.x);
   const int bh = work / nqt, h = bh % a.H, b = bh / a.H;
   const int t = threadIdx.x;
   F32Args f;
@@ -538,13 +539,17 @@ static int rpb_f32_launch(RpbArgs& a, int mode, hipStream_t st, const char* name
   }
   const size_t lds = (size_t)a.lut_len * 4;
 #define VFK_RPB_F32(M, C) \
-  hipLaunchKernelGGL((rpb_fwd_f32_kernel<M, C>), dim3((unsigned)grid), dim3(256), lds, st, a)
+  hipLaunchKernelGGL((rpb_fwd_f32_kernel<M, C>), dim3(n), dim3(256), lds, st, a)
 #define VFK_RPB_F32_M(M) \
   if (a.causal) VFK_RPB_F32(M, true); else VFK_RPB_F32(M, false);
-  switch (mode) {
-    case MASK_NONE: VFK_RPB_F32_M(MASK_NONE) break;
-    case MASK_KEY: VFK_RPB_F32_M(MASK_KEY) break;
-    default: VFK_RPB_F32_M(MASK_FULL) break;
+  for (int64_t w0 = 0; w0 < grid; w0 += kF32MaxGrid) {
+    const unsigned n = (unsigned)std::min(kF32MaxGrid, grid - w0);
+    a.work0 = (int)w0;
+    switch (mode) {
+      case MASK_NONE: VFK_RPB_F32_M(MASK_NONE) break;
+      case MASK_KEY: VFK_RPB_F32_M(MASK_KEY) break;
+      default: VFK_RPB_F32_M(MASK_FULL) break;
+    }
   }
 #undef VFK_RPB_F32_M
 #undef VFK_RPB_F32
