@@ -146,3 +146,17 @@ def test_glu_linear_row_alone_and_among_others(dev):
         got, want = glu_linear(x[:n], w, "gelu").float(), full[:n].float()
         step = torch.maximum(got.abs(), want.abs()) * 2 ** -7  # a bf16 step is at most 2^-7 of the value
         assert ((got - want).abs() <= step + 1e-4).all(), n
+
+
+@pytest.mark.parametrize("at", [0, 1, 4, 8])
+@pytest.mark.parametrize("pad", [1, 3, 8])
+def test_glu_linear_single_row_of_any_stride(dev, at, pad):
+    """One row cut out of a wider one, at any offset and with any stride to a
+    row that is not there: the same bits as the row by itself."""
+    from kernels.fused_glu_mlp import glu_linear
+    x, w = _inputs(1, 256, 64, torch.bfloat16, 5)
+    buf = torch.zeros(1, 256 + at + pad, dtype=torch.bfloat16, device=dev)
+    buf[:, at:at + 256] = x.to(dev)
+    cut = buf[:, at:at + 256]
+    got = glu_linear(cut, w.to(dev), "gelu")
+    assert got.shape == (1, 64) and torch.equal(got, glu_linear(x.to(dev), w.to(dev), "gelu"))

@@ -55,7 +55,8 @@ def glu_linear(x: torch.Tensor, weight: torch.Tensor, act_fn: str = "gelu",
     if weight.dtype != x.dtype:
         raise ValueError("glu_linear: x and weight must share a dtype")
     I = weight.shape[0] // 2
-    x2 = _lib.rows_aligned(x if x.dim() == 2 else x.reshape(-1, K))
+    # a single row may have any row stride: the reshape makes it K
+    x2 = _lib.rows_aligned(x if x.dim() == 2 and x.shape[0] != 1 else x.reshape(-1, K))
     w2 = _lib.rows_aligned(weight)
     if out is None:
         out = x.new_empty((x2.shape[0], I))
