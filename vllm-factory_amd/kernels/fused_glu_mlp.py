@@ -49,14 +49,15 @@ def glu_linear(x: torch.Tensor, weight: torch.Tensor, act_fn: str = "gelu",
     (up to 224 at I = 1152) split K over four waves: such a row agrees with
     itself among more rows to rounding, from there on bit for bit."""
     dev = _lib.require_gpu(x, weight)
-    K = x.shape[-1]
+    shape = x.shape
+    K = shape[-1]
     if weight.dim() != 2 or weight.shape[1] != K or weight.shape[0] % 2:
         raise ValueError(f"glu_linear: weight must be [2I, {K}], got {tuple(weight.shape)}")
     if weight.dtype != x.dtype:
         raise ValueError("glu_linear: x and weight must share a dtype")
     I = weight.shape[0] // 2
     # a single row may have any row stride: the reshape makes it K
-    x2 = _lib.rows_aligned(x if x.dim() == 2 and x.shape[0] != 1 else x.reshape(-1, K))
+    x2 = _lib.rows_aligned(x if len(shape) == 2 and shape[0] != 1 else x.reshape(-1, K))
     w2 = _lib.rows_aligned(weight)
     if out is None:
         out = x.new_empty((x2.shape[0], I))
@@ -64,4 +65,4 @@ def glu_linear(x: torch.Tensor, weight: torch.Tensor, act_fn: str = "gelu",
         raise ValueError(f"glu_linear: out must be [{x2.shape[0]}, {I}] {x.dtype}")
     _lib.on_device("vfk_glu_linear_fwd", dev, _act_code(act_fn), _lib.ref(_lib.desc(x2)),
                    _lib.ref(_lib.desc(w2)), _lib.ref(_lib.desc(out)))
-    return out if x.dim() == 2 else out.view(*x.shape[:-1], I)
+    return out if len(shape) == 2 else out.view(*shape[:-1], I)

@@ -16,7 +16,8 @@ from . import _lib
 
 def _as_2d(x: torch.Tensor, n: int) -> torch.Tensor:
     # a single row may have any row stride: the reshape makes it n
-    x2 = x if x.dim() == 2 and x.shape[1] == n and x.shape[0] != 1 else x.reshape(-1, n)
+    s = x.shape
+    x2 = x if len(s) == 2 and s[1] == n and s[0] != 1 else x.reshape(-1, n)
     if x2.stride(-1) != 1:
         x2 = x2.contiguous()
     return x2
